@@ -65,6 +65,7 @@ struct SideTables {
     WaveUnit *units = nullptr;
     double *preflog = nullptr, *tref = nullptr;  // SW
     LwConst *cst = nullptr;                      // LW
+    LwBand *bands_fwd = nullptr;                 // LW: the same for the forward kernel's copy
     LwBand *bands_lds = nullptr;                 // LW: offsets relative to each band's first k-table element
     LwLdsPlan plan{};                            // LW: schedule of the LDS-table kernel
     bool lds = false;                            // LW: that kernel fits this device
@@ -387,7 +388,7 @@ int rrtmg_hip_sw_init(double cpdair, const char *table_dir)
 // are one contiguous range of the packed buffer (tables.cpp packs them band
 // by band, before the transmittance tables); every k-table offset of the band
 // must lie in it, and is rebased to its start for the LDS copy.
-static bool make_lw_plan(const LwHost &h, LwLdsPlan &p, LwBand *rebased, std::string &err)
+static bool make_lw_plan(const LwHost &h, LwLdsPlan &p, LwBand *rebased, LwBand *fwd, std::string &err)
 {
     for (int b = 0; b < 16; ++b) {
         const LwBand &d = h.tab.band[b];
@@ -421,6 +422,19 @@ static bool make_lw_plan(const LwHost &h, LwLdsPlan &p, LwBand *rebased, std::st
             *f -= lo;
         }
         rebased[b] = r;
+        // the forward kernel's copy: absb of bands 3-5 left out, its offset global
+        p.cut0[b] = p.cut1[b] = hi - lo;
+        if (b >= 2 && b <= 4) {
+            const int rows = 47 * 5 * LW_NSPB[b];
+            p.cut0[b] = r.absb;
+            p.cut1[b] = r.absb + (rows * lw_ng(b + 1) + 3) / 4 * 4;
+            for (int *f : fields)
+                if (*f >= p.cut1[b]) *f -= p.cut1[b] - p.cut0[b];
+            r.absb = h.tab.band[b].absb;
+        }
+        fwd[b] = r;
+        const int et = (int)((2 * (NTBL + 1) * sizeof(float) + 15) / 16 * 16);
+        p.fwd_lds_bytes = std::max(b ? p.fwd_lds_bytes : 0, et + (int)sizeof(float) * (hi - lo - (p.cut1[b] - p.cut0[b]) + 4));
         p.ubeg[b] = -1;
         p.upt[b] = 0;
     }
@@ -461,9 +475,10 @@ int rrtmg_hip_lw_init(double cpdair, const char *table_dir)
     if (!rc) rc = upload((LwBand **)&s->lwd.bands, s->lw.tab.band, sizeof s->lw.tab.band);
     if (!rc) rc = upload(&s->lwd.units, s->lw.units.data(), s->lw.units.size() * sizeof(WaveUnit));
     if (!rc) rc = upload(&s->lwd.cst, &s->lw.cst, sizeof(LwConst));
-    LwBand rebased[16];
-    if (!rc && !make_lw_plan(s->lw, s->lwd.plan, rebased, err)) return fail(RRTMG_HIP_ENOENT, err);
+    LwBand rebased[16], fwd[16];
+    if (!rc && !make_lw_plan(s->lw, s->lwd.plan, rebased, fwd, err)) return fail(RRTMG_HIP_ENOENT, err);
     if (!rc) rc = upload(&s->lwd.bands_lds, rebased, sizeof rebased);
+    if (!rc) rc = upload(&s->lwd.bands_fwd, fwd, sizeof fwd);
     {
         // optional: the water-path cloud optics' coefficients (inflglw 1, 2)
         TableFile ct;
@@ -488,7 +503,7 @@ int rrtmg_hip_lw_init(double cpdair, const char *table_dir)
         if (lds_device(&ncu, &lds)) return fail(RRTMG_HIP_EDEVICE, "device attribute query failed");
         s->lwd.plan.ncu = ncu;
         const char *env = std::getenv("RRTMG_HIP_LW_LDS");
-        s->lwd.lds = s->lwd.plan.lds_bytes <= lds && !(env && env[0] == '0');
+        s->lwd.lds = std::max(s->lwd.plan.lds_bytes, s->lwd.plan.fwd_lds_bytes + 64) <= lds && !(env && env[0] == '0');
     }
     s->lwd.cpdair = cpdair;
     s->lwd.ready = true;
@@ -923,7 +938,6 @@ static int lw_forward(int ncol, int nlay, int icld, int idrv, const double *play
     }
     const int mixed = g_prec == RRTMG_HIP_PREC_MIXED;
     const size_t rs = mixed ? sizeof(float) : sizeof(double);
-    if ((rc = check_lds(lw_fwd_lds_bytes(nlay, rs)))) return rc;
     int ck = 0;
     size_t off = 0;
     const size_t o_coef = off; off = align_up(off + rs * LWF_STRIDE * n2);
@@ -932,14 +946,13 @@ static int lw_forward(int ncol, int nlay, int icld, int idrv, const double *play
     const size_t o_ilev = off; off = align_up(off + sizeof(int) * n3);
     const size_t o_lt = off; off = align_up(off + sizeof(int) * ncol);
     const size_t o_cs = off; off = align_up(off + sizeof(double) * 3 * ncol);
-    const size_t o_bf = off; off = align_up(off + rs * 16 * 2 * n3);
-    const int chunk = vjp_chunk((ncol + TILE_COLS - 1) / TILE_COLS * s->lw.tab.nwaves, lw_fwd_state_bytes(nlay, rs));
+    const size_t o_bf = off; if (!cloudy) off = align_up(off + rs * 16 * 2 * n3);
     const bool lds = mixed && s->lwd.lds;
-    const size_t ds_bytes = lds ? (size_t)lw_lds_grid(s->lwd.plan, ncol, s->lw.tab.nwaves) * LW_WGW *
-                                      lw_lds_state_bytes(nlay)
-                                : (size_t)chunk * lw_fwd_state_bytes(nlay, rs);
-    const size_t o_ds = off; off = align_up(off + ds_bytes);
-    const size_t o_it = off; off = align_up(off + sizeof(int));
+    const int kind = lw_fwd_kind(ncol, rs, s->lwd.plan.ncu, lds, g_prec == RRTMG_HIP_PREC_FP64_SMOOTH);
+    const int chunk = lw_fwd_grid(ncol, nlay, rs, s->lwd.plan.ncu, kind);
+    const size_t o_ds = off;
+    if (!cloudy) off = align_up(off + (size_t)chunk * lw_fwd_rows_bytes(nlay, rs, kind));
+    const size_t o_it = off; off = align_up(off + 8 * sizeof(int));
     // cloud path: flags, overlap records, four-stream band fluxes, scratch rows
     const int cchunk = vjp_chunk((ncol + TILE_COLS - 1) / TILE_COLS * s->lw.tab.nwaves, lw_cloud_row_bytes(nlay, rs));
     const size_t o_cfl = off; if (cloudy) off = align_up(off + sizeof(int) * n2);
@@ -962,6 +975,7 @@ static int lw_forward(int ncol, int nlay, int icld, int idrv, const double *play
     w.dstate = wb + o_ds;
     w.chunk = chunk;
     w.items = (int *)(wb + o_it);
+    w.kind = kind;
     LwCloudWork cw;
     LwClouds cld{};
     if (cloudy) {
@@ -1056,6 +1070,7 @@ static int lw_forward(int ncol, int nlay, int icld, int idrv, const double *play
     t.units = s->lwd.units;
     t.heatfac = s->lw.cst.heatfac;
     t.bands_lds = s->lwd.bands_lds;
+    t.bands_fwd = s->lwd.bands_fwd;
     t.plan = s->lwd.plan;
     t.lds = lds;
     if (ck) return fail(RRTMG_HIP_EDEVICE, "LW: host-to-device copy failed");

@@ -2,6 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "../../include/rrtmg_hip.h"
 #include "rrtmg_types.hpp"
 
@@ -47,9 +49,10 @@ struct LwWork {
     int *laytrop = nullptr;   // [ncol]
     double *colscal = nullptr;// [3][ncol]: pwvcm, tbound, (spare)
     void *bflux = nullptr;    // [16][2][nlay+1][ncol] of Real
-    void *dstate = nullptr;   // [chunk][nlay][64] of Real: upward source of each wave of a band-kernel launch
-    int chunk = 0;            // wave units per band-kernel launch (rows of dstate)
-    int *items = nullptr;     // work-item counter of the LDS-table band kernel
+    void *dstate = nullptr;   // [chunk][waves] scratch rows, lw_fwd_state_bytes each
+    int chunk = 0;            // workgroups of the band kernel
+    int *items = nullptr;     // work-item counters of the persistent band kernels, 8
+    int kind = 0;             // which band kernel (lw_fwd_kind)
 };
 
 struct SwDevTables {
@@ -70,6 +73,10 @@ struct LwLdsPlan {
     int ubeg[16];   // first unit of each band in a tile's unit list
     int upt[16];    // units of each band per tile
     int lds_bytes;  // largest band's k-tables in FP32
+    // the forward kernel's LDS copy leaves [cut0, cut1) of a band's k-tables
+    // out (absb of the bands whose tables exceed what the exp and transition
+    // tables leave); its LDS in bytes
+    int cut0[16], cut1[16], fwd_lds_bytes;
     int ncu;        // compute units: workgroups of one launch
 };
 // rows of per-wave global scratch (transmittance and upward source, nlay x 64
@@ -99,6 +106,7 @@ struct LwDevTables {
     const LwConst *cst;       // device copy
     const WaveUnit *units;
     double heatfac;
+    const LwBand *bands_fwd = nullptr;  // the same for the forward kernel's copy (absb global where left out)
     const LwBand *bands_lds = nullptr;  // desc.band with k-table offsets relative to the band's first element
     LwLdsPlan plan{};
     bool lds = false;                   // FP32 forward uses the LDS-table kernel
@@ -285,7 +293,8 @@ struct LwVjpWork {
                               // ([rows][3][nlay][64] with the transmittance for the LDS-table kernel)
     int chunk = 0;            // wave units per backward band-kernel launch (rows of dstate)
     void *bflux = nullptr;    // [16][2][nlay+1][ncol] of Real: band fluxes of the recomputed forward, or NULL
-    int *items = nullptr;     // work-item counter of the LDS-table band kernel
+    int *items = nullptr;     // work-item counters of the persistent band kernels, 8
+    int kind = 0;             // which band kernel (lw_fwd_kind)
 };
 struct SwVjpWork {
     void *dcoef = nullptr;    // [nlay][ncol][SWF_STRIDE] of Real: the field values
@@ -312,9 +321,49 @@ inline int vjp_chunk(int units, size_t bytes_per_unit)
     return units < (int)c ? units : (int)c;
 }
 inline size_t sw_fwd_state_bytes(int nlay, size_t real_size) { return real_size * 2 * (size_t)(nlay + 1) * 64; }
-inline size_t lw_fwd_state_bytes(int nlay, size_t real_size) { return real_size * (size_t)nlay * 64; }
+// LW forward: the optical depths of a lane's g-points, up to four
+inline size_t lw_fwd_state_bytes(int nlay, size_t real_size) { return real_size * 4 * (size_t)nlay * 64; }
+// and of its form that shares the layers of a unit among the waves of a
+// workgroup: the transmittances, two sources and the radiances of each
+inline size_t lw_fwd_layers_bytes(int nlay, size_t real_size) { return real_size * 4 * (4 * (size_t)nlay + 1) * 64; }
+// units of work of the LW forward: CPW columns of a band
+inline size_t lw_fwd_units(int ncol)
+{
+    size_t n = 0;
+    for (int b = 1; b <= 16; ++b) n += ((size_t)ncol + lw_cpw(b) - 1) / lw_cpw(b);
+    return n;
+}
+// the LW forward kernel: 16 lw_band_lds_kernel (FP32, lds: its tables fit the
+// device); 8 lw_band_kernel with a wave per unit (FP64, and the smooth mode,
+// which has no tables to read from L2); 1 and 2 with a workgroup of eight or of
+// four waves per unit.  Below 4096 columns the latter two are the faster (FP32
+// 2261 x 59: 309 us against 345 of the LDS kernel; FP64 2048 x 40: 339 against
+// 410 of a wave per unit), above it the slower (8192 x 40: FP32 663 against
+// 374, FP64 1206 against 843); eight waves where one workgroup per unit does
+// not fill the chip (128 x 40: 56 us against 176 of a wave per unit).
+inline int lw_fwd_kind(int ncol, size_t real_size, int ncu, bool lds, bool smooth)
+{
+    if (smooth) return 8;
+    if (lw_fwd_units(ncol) <= (size_t)ncu) return 1;
+    if (ncol < 4096) return 2;
+    return real_size == 4 ? (lds ? 16 : 2) : 8;
+}
+// scratch rows of a workgroup
+inline size_t lw_fwd_rows_bytes(int nlay, size_t real_size, int kind)
+{
+    return kind < 8 ? lw_fwd_layers_bytes(nlay, real_size) : kind * lw_fwd_state_bytes(nlay, real_size);
+}
+// its workgroups: those that fit the chip at once, no more than there is work
+// for or than 2 GiB of rows hold
+inline int lw_fwd_grid(int ncol, int nlay, size_t real_size, int ncu, int kind)
+{
+    const size_t rows = VJP_SCRATCH_BYTES / lw_fwd_rows_bytes(nlay, real_size, kind);
+    const size_t items = kind == 16  ? ((size_t)ncol + LW_TILE - 1) / LW_TILE * LW_TILE_ITEMS
+                         : kind == 8 ? (lw_fwd_units(ncol) + 7) / 8
+                                     : lw_fwd_units(ncol);
+    return (int)std::max<size_t>(1, std::min({rows, items, (size_t)ncu * (kind == 2 ? 2 : 1)}));
+}
 inline size_t sw_fwd_lds_bytes(int, size_t real_size) { return real_size * 64; }
-inline size_t lw_fwd_lds_bytes(int nlay, size_t real_size) { return real_size * ((size_t)nlay * 64 + 64); }
 __host__ __device__ inline size_t sw_vjp_state_bytes(int nlay, size_t real_size)
 {
     return real_size * (4 * (size_t)(nlay + 1) + 5 * (size_t)nlay) * 64;

@@ -2,27 +2,33 @@
 // rtrnmr per g-point) and finish (band sums, fluxfac, heating).  Reference:
 // rrtmg_lw/gcm_model/src/ of MiMA's RRTMG_LW (file:line cited per function).
 //
-// Band kernel: one wave per work unit (band b, up to 64/ng columns of a
-// tile), lane = (column, g).  Each band is a compile-time instantiation, so a
-// wave runs straight-line band code.  Per lane: a downward sweep computes the
-// layer optical depth and Planck fraction, the transmittance and source
-// (table or thin-layer series) and the downward radiance, keeping
-// (atrans, bbugas) per layer in LDS; the surface term and an upward sweep
-// follow.  Radiances are summed over the band's g-points of a column
-// (segmented sum over ng adjacent lanes) into per-band level fluxes.
-// FP32 runs the same body in lw_band_lds_kernel: persistent 16-wave
-// workgroups that copy one band's k-tables (at most 128 KB) into LDS, so the
-// ~30 k-table gathers per layer take LDS latency rather than L2 latency
-// (64-lane gathers across four columns miss the 32 KB L1); a 16-wave
-// workgroup also holds the kernel at 128 VGPRs, four waves per SIMD.  FP64
-// (whose bands 3-5 exceed 160 KB of LDS) and RRTMG_HIP_LW_LDS=0 use
-// lw_band_kernel, one wave per workgroup.
+// Band kernels: a lane holds up to four g-points of one column, LPC adjacent
+// lanes a band, CPW columns a wave (LwLanes).  The gas optics are weighted table
+// rows (lw_rows.hpp), so what does not depend on the g-point (coefficients,
+// species parameters, weights, Planck values) is formed once for four
+// g-points, a table row is one 16-byte load, and the g-sum is three additions
+// and at most two shuffles.  With one g-point per lane the same work took twice
+// the instructions (32768 columns x 40 layers: 2.16 ms -> 1.11 ms in FP32,
+// 8192 x 40 in FP64: 1.35 -> 0.83 ms).
+//
+// Three kernels, by the size of the call (lw_fwd_kind); a column's result is
+// the same bits in each:
+// * lw_band_lds_kernel, large FP32 calls: what bounds it is LDS and L1
+//   bandwidth (every optical depth takes about 18 table values), so the (exp,
+//   transition function) pairs, 80 KB, and the k-tables of the workgroup's band
+//   are in LDS; VALU 50% of its time.
+// * lw_band_kernel, a wave per unit, large FP64 calls: the FP64 pairs alone
+//   take 160 KB of LDS, the k-tables come from L1 and L2.
+// * lw_band_kernel, a workgroup per unit with its waves sharing the layers,
+//   calls below 4096 columns: too few waves to hide a layer's chain of
+//   dependent loads (128 x 40: 137 -> 56 us).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 
 #include "kernels.hpp"
 #include "lw_optics.hpp"
+#include "lw_rows.hpp"
 #include "rrtmg_device.hpp"
 
 namespace rrtmg {
@@ -37,11 +43,8 @@ __global__ __launch_bounds__(256) void lw_prep_kernel(ColumnInputs in, LwWork w,
 {
     const int ncol = in.ncol, nlay = in.nlay;
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t n = (size_t)nlay * ncol, iblk = (size_t)blockIdx.x * blockDim.x;
+    const size_t n = (size_t)nlay * ncol;
     const int lay = (int)(i / ncol), col = (int)(i - (size_t)lay * ncol);
-    // this thread's coefficient record, staged for store_records
-    __shared__ __align__(16) Real srec[256 * LWF_STRIDE];
-    Real *rec = srec + threadIdx.x * LWF_STRIDE;
     Real *tlevf = (Real *)w.tlev;
     const double amd = 28.9660, amw = 18.0160, amdw = 1.607793, amdo = 0.603428;
     const double avogad = 6.02214199e+23, grav = 9.8066;
@@ -130,6 +133,7 @@ __global__ __launch_bounds__(256) void lw_prep_kernel(ColumnInputs in, LwWork w,
         if (colch4 == 0.0) colch4 = 1.e-32 * coldry;
         double colbrd = 1.e-20 * wbrodl;
         double compfp = 1. - fp;
+        Real rec[LWF_STRIDE];
         rec[LWF_FAC10] = (Real)(compfp * ft);
         rec[LWF_FAC00] = (Real)(compfp * (1.0 - ft));
         rec[LWF_FAC11] = (Real)(fp * ft1);
@@ -158,9 +162,15 @@ __global__ __launch_bounds__(256) void lw_prep_kernel(ColumnInputs in, LwWork w,
         rec[LWF_TLAYFRAC] = (Real)tlayfrac;
         w.ipk[ix] = pack_lw(jp, jt, jt1, indself, indfor, indminor, indlay);
         for (int f = LWF_COUNT; f < LWF_STRIDE; ++f) rec[f] = (Real)0;
+        // [lay][group][col][4]: a wave's store of a group is contiguous
+        struct alignas(16) Group {
+            Real x[4];
+        };
+        Group *g = (Group *)w.coef + (size_t)lay * LWF_GROUPS * ncol + col;
+#pragma unroll
+        for (int k = 0; k < LWF_GROUPS; ++k)
+            g[(size_t)k * ncol] = {rec[4 * k], rec[4 * k + 1], rec[4 * k + 2], rec[4 * k + 3]};
     }
-    const int nrec = (int)(n - iblk < blockDim.x ? n - iblk : blockDim.x);
-    store_records<Real, LWF_STRIDE>((Real *)w.coef + iblk * LWF_STRIDE, srec, nrec);
 }
 
 // per-column part of the prep (one thread per column): laytrop and the
@@ -193,203 +203,423 @@ __global__ __launch_bounds__(256) void lw_column_kernel(ColumnInputs in, LwWork 
     w.colscal[(size_t)ncol + col] = in.tsfc[col];
 }
 
-// One band of one work unit (rrtmg_lw_rtrnmr.f90:483-716, clear sky).
-// ktab: the k-tables (B's offsets index it; the packed global buffer, or the
-// band's copy in LDS with rebased offsets); tab: the packed global buffer
-// (transmittance and Planck tables).  s_atr, s_bbu: transmittance and upward
-// source per layer, [nlay][64] each (LDS or this wave's global scratch row);
-// s_red: 64 LDS entries for the FP64 g-sum.
+// contraction off, as in lw_rows.hpp
+#pragma clang fp contract(off)
+
+// Sum of a column's g-points on its first lane: exact enough in FP64 (the sum
+// is rounded once to FP32, and FP64 differs from the reference's order by its
+// last digits only).
 template <int BAND, typename Real>
-__device__ __forceinline__ void lw_band_body(const ColumnInputs &in, const LwWork &w, const LwBand &B, const Real *__restrict__ ktab,
-                             const Real *__restrict__ tab, int exp_off, int tfn_off, int plk_off,
-                             const LwConst *__restrict__ cst, WaveUnit u, int tile, int lane,
-                             Real *__restrict__ s_atr, Real *__restrict__ s_bbu, Real *s_red)
+__device__ __forceinline__ Real band_sum(const Real (&v)[LwLanes<BAND>::GC], int g0)
 {
-    constexpr int NG = lw_ng(BAND);
-    const int ncol = in.ncol, nlay = in.nlay;
-    const int cl = lane / NG, g = lane - cl * NG;
-    const GSum<Real, NG> gsum(lane, g);
-    const int col0 = tile * TILE_COLS + u.first_col + cl;
-    const bool active = cl < u.ncols && col0 < ncol;
-    const int col = active ? col0 : 0;
-    const Real *coef = (const Real *)w.coef;
-    const Real *tlevf = (const Real *)w.tlev;
-    const Real *exp_tbl = exp_off >= 0 ? tab + exp_off : nullptr;
-    const Real *tfn_tbl = tfn_off >= 0 ? tab + tfn_off : nullptr;
-    const Real *plk = tab + plk_off + (BAND - 1) * 181;  // totplnk(:, BAND)
-    LTab<Real> T{ktab, NG, g};
-    Real *bf_up = (Real *)w.bflux + (size_t)(BAND - 1) * 2 * (nlay + 1) * ncol;
-    Real *bf_dn = bf_up + (size_t)(nlay + 1) * ncol;
-
-    const int laytrop = w.laytrop[col];
-    const double pwvcm = w.colscal[col];
-    const double tbound = w.colscal[(size_t)ncol + col];
-    // diffusivity secant (rrtmg_lw_rtrnmr.f90:272-280)
-    double sd = 1.66;
-    if (!(BAND == 1 || BAND == 4 || BAND >= 10)) {
-        sd = B.a0 + B.a1 * exp(B.a2 * pwvcm);
-        if (sd > 1.80) sd = 1.80;
-        if (sd < 1.50) sd = 1.50;
+    using L = LwLanes<BAND>;
+    double s = 0.0;
+#pragma unroll
+    for (int j = 0; j < L::GC; ++j) {
+        const bool in = L::NG % L::GC == 0 || g0 + j < L::NG;
+        s = j == 0 ? (double)v[0] : in ? s + (double)v[j] : s;
     }
-    const Real secdiff = (Real)sd;
-    const Real semiss = (Real)in.emis[(size_t)(BAND - 1) * ncol + col];
-    // surface Planck (rrtmg_lw_setcoef.f90:190-194), FP64
-    int indbound = clampi((int)(tbound - 159.0), 1, 180);
-    double tbndfrac = tbound - 159.0 - (double)indbound;
-    const Real plankbnd =
-        (Real)((double)semiss * ((double)plk[indbound - 1] + tbndfrac * ((double)plk[indbound] - (double)plk[indbound - 1])));
-    auto planklev = [&](int lev) {
-        int i = at32(w.ilev, (unsigned)(lev * ncol + col));
-        Real f = at32(tlevf, (unsigned)(lev * ncol + col));
-        return at32(plk, (unsigned)(i - 1)) + f * (at32(plk, (unsigned)i) - at32(plk, (unsigned)(i - 1)));
-    };
-    const double *tauaer = in.tauaer;
-
-    // downward sweep
-    Real radld = (Real)0, fracs1 = (Real)0;
-    Real plev_up = planklev(nlay);
-    if (active && g == 0) at32(bf_dn, (unsigned)(nlay * ncol + col)) = (Real)0;  // drad(nlayers) stays 0
-    LwLayer<Real> c;
-    for (int lev = nlay; lev >= 1; --lev) {
-        lw_load_layer(c, coef, w.ipk, lev - 1, col, ncol, nlay);
-        Real taug, plfrac;
-        lw_gas<BAND, Real, Real, true>(B, T, cst, c, lev <= laytrop, taug, plfrac);
-        if (tauaer) taug = taug + (Real)tauaer[((size_t)(BAND - 1) * nlay + (lev - 1)) * ncol + col];
-        Real plev_dn = planklev(lev - 1);
-        Real blay = at32(plk, (unsigned)(c.indlay - 1)) +
-                    c.tlayfrac * (at32(plk, (unsigned)c.indlay) - at32(plk, (unsigned)(c.indlay - 1)));
-        Real dplankup = plev_up - blay, dplankdn = plev_dn - blay;
-        Real odepth = secdiff * taug;
-        if (odepth < (Real)0) odepth = (Real)0;
-        Real atrans, bbd, bbugas;
-        if (!exp_tbl) {  // smooth mode: the tabulated functions at every depth
-            const LwRT<Real> rt = lw_rt_exact(odepth, false);
-            atrans = rt.atrans;
-            bbd = plfrac * (blay + rt.tf * dplankdn);
-            bbugas = plfrac * (blay + rt.tf * dplankup);
-        } else if (odepth <= (Real)0.06) {
-            atrans = odepth - (Real)0.5 * odepth * odepth;
-            odepth = (Real)0.166667 * odepth;
-            bbd = plfrac * (blay + dplankdn * odepth);
-            bbugas = plfrac * (blay + dplankup * odepth);
-        } else {
-            const int itr = tbl_index(odepth);
-            atrans = (Real)1 - at32(exp_tbl, (unsigned)itr);
-            const Real tausfac = at32(tfn_tbl, (unsigned)itr);
-            bbd = plfrac * (blay + tausfac * dplankdn);
-            bbugas = plfrac * (blay + tausfac * dplankup);
-        }
-        radld = radld + (bbd - radld) * atrans;
-        at32(s_atr, (unsigned)((lev - 1) * 64 + lane)) = atrans;
-        at32(s_bbu, (unsigned)((lev - 1) * 64 + lane)) = bbugas;
-        Real s = gsum.sum(active ? radld : (Real)0, s_red);
-        if (active && g == 0) at32(bf_dn, (unsigned)((lev - 1) * ncol + col)) = s;
-        plev_up = plev_dn;
-        if (lev == 1) fracs1 = plfrac;
+    if constexpr (L::LPC == 2) s = s + __shfl_down(s, 1);
+    if constexpr (L::LPC == 3) s = s + (__shfl_down(s, 1) + __shfl_down(s, 2));
+    if constexpr (L::LPC == 4) {
+        s = s + __shfl_down(s, 1);
+        s = s + __shfl_down(s, 2);
     }
-    // surface emission and reflection, upward sweep
-    Real radlu = fracs1 * plankbnd + ((Real)1 - semiss) * radld;
+    return (Real)s;
+}
+
+// (exp(-tau), tau transition function) entries of the 10000-interval tables
+template <typename Real>
+struct alignas(2 * sizeof(Real)) ExpTfn {
+    Real e, t;
+};
+
+// What a wave needs of one band and CPW columns from column c0 on, below cend.
+// ktab: the band's k-tables, at B's offsets (global, or a copy in LDS); ktab_b:
+// those of the upper atmosphere's major species (absb); tab: the packed global
+// buffer (Planck); et: the (exp, tfn) pairs (global or LDS), or NULL for the
+// smooth functions.
+template <int BAND, typename Real>
+struct LwUnit {
+    using L = LwLanes<BAND>;
+    static constexpr int NG = L::NG, GC = L::GC;
+    const ColumnInputs &in;
+    const LwWork &w;
+    const LwBand &B;
+    const Real *__restrict__ ktab, *__restrict__ ktab_b, *__restrict__ plk;
+    const ExpTfn<Real> *et;
+    const LwConst *__restrict__ cst;
+    int g0, col, laytrop;
+    bool first;  // the lane that stores the column's sums
+    Real secdiff;
+    __device__ __forceinline__ LwUnit(const ColumnInputs &in_, const LwWork &w_, const LwBand &B_,
+                                      const Real *ktab_, const Real *ktab_b_, const Real *tab,
+                                      const ExpTfn<Real> *et_, int plk_off, const LwConst *cst_, int c0, int cend,
+                                      int lane)
+        : in(in_), w(w_), B(B_), ktab(ktab_), ktab_b(ktab_b_), plk(tab + plk_off + (BAND - 1) * 181), et(et_), cst(cst_)
     {
-        Real s = gsum.sum(active ? radlu : (Real)0, s_red);
-        if (active && g == 0) at32(bf_up, (unsigned)col) = s;
+        const int cl = lane / L::LPC;
+        g0 = (lane - cl * L::LPC) * GC;
+        const bool active = cl < L::CPW && c0 + cl < cend;
+        col = active ? c0 + cl : cend - 1;
+        first = active && g0 == 0;
+        laytrop = w.laytrop[col];
+        // diffusivity secant (rrtmg_lw_rtrnmr.f90:272-280)
+        double sd = 1.66;
+        if (!(BAND == 1 || BAND == 4 || BAND >= 10)) {
+            sd = B.a0 + B.a1 * exp(B.a2 * w.colscal[col]);
+            if (sd > 1.80) sd = 1.80;
+            if (sd < 1.50) sd = 1.50;
+        }
+        secdiff = (Real)sd;
     }
-    // the per-layer states are read four levels ahead (rotating registers),
-    // so a level's load has three levels of work to complete behind
-    auto at = [&](const Real *p, int i) { return i < nlay ? at32(p, (unsigned)(i * 64 + lane)) : (Real)0; };
-    Real b0 = at(s_bbu, 0), b1 = at(s_bbu, 1), b2 = at(s_bbu, 2), b3 = at(s_bbu, 3);
-    Real a0 = at(s_atr, 0), a1 = at(s_atr, 1), a2 = at(s_atr, 2), a3 = at(s_atr, 3);
+    __device__ __forceinline__ void load(LwLayer<Real> &c, int lev) const
+    {
+        lw_load_layer(c, (const Real *)w.coef, w.ipk, lev - 1, col, in.ncol, in.nlay);
+    }
+    __device__ __forceinline__ Real planklev(int lev) const
+    {
+        const int i = at32(w.ilev, (unsigned)(lev * in.ncol + col));
+        const Real f = at32((const Real *)w.tlev, (unsigned)(lev * in.ncol + col));
+        return fma(f, at32(plk, (unsigned)i) - at32(plk, (unsigned)(i - 1)), at32(plk, (unsigned)(i - 1)));
+    }
+    __device__ __forceinline__ Real planklay(const LwLayer<Real> &c) const
+    {
+        return fma(c.tlayfrac, at32(plk, (unsigned)c.indlay) - at32(plk, (unsigned)(c.indlay - 1)),
+                   at32(plk, (unsigned)(c.indlay - 1)));
+    }
+    // optical depths on the diffusivity path of layer lev, from its record
+    __device__ __forceinline__ void depths(const LwLayer<Real> &c, int lev, Real (&od)[GC]) const
+    {
+        const bool lower = lev <= laytrop;
+#pragma unroll
+        for (int j = 0; j < GC; ++j) od[j] = (Real)0;
+        lw_rows<BAND, Real, Real>(B, cst, c, lower, [&](auto where, int off, int r, Real wt) {
+            Real k[GC];
+            load_row<NG>(k, where == LW_ABSB ? ktab_b : ktab, (unsigned)(off + (r - 1) * NG + g0));
+#pragma unroll
+            for (int j = 0; j < GC; ++j) od[j] = fma(wt, k[j], od[j]);
+        });
+        const Real ta =
+            in.tauaer ? (Real)in.tauaer[((size_t)(BAND - 1) * in.nlay + (lev - 1)) * in.ncol + col] : (Real)0;
+#pragma unroll
+        for (int j = 0; j < GC; ++j) {
+            if constexpr (BAND == 4 || BAND == 7) od[j] = od[j] * lw_gfactor<BAND, Real>(g0 + j, lower);
+            od[j] = secdiff * (od[j] + ta);
+            if (od[j] < (Real)0) od[j] = (Real)0;
+        }
+    }
+    // Planck fractions of layer lev
+    __device__ __forceinline__ void fracs(const LwLayer<Real> &c, int lev, Real (&fr)[GC]) const
+    {
+#pragma unroll
+        for (int j = 0; j < GC; ++j) fr[j] = (Real)0;
+        lw_fracs<BAND, Real, Real>(B, cst, c, lev <= laytrop, [&](int off, int r, Real wt) {
+            Real k[GC];
+            load_row<NG>(k, ktab, (unsigned)(off + (r - 1) * NG + g0));
+#pragma unroll
+            for (int j = 0; j < GC; ++j) fr[j] = fma(wt, k[j], fr[j]);
+        });
+    }
+    // transmittance and transition function of an optical depth
+    __device__ __forceinline__ void transmit(Real od, Real &atr, Real &tf) const
+    {
+        if (!et) {  // smooth mode: the tabulated functions at every depth
+            const LwRT<Real> rt = lw_rt_exact(od, false);
+            atr = rt.atrans;
+            tf = rt.tf;
+        } else {
+            const ExpTfn<Real> x = et[tbl_index(od)];
+            const bool thin = od <= (Real)0.06;
+            atr = thin ? fma((Real)-0.5 * od, od, od) : (Real)1 - x.e;
+            tf = thin ? (Real)0.166667 * od : x.t;
+        }
+    }
+    // surface emission and reflection: downward radiances into upward ones
+    __device__ __forceinline__ void surface(const Real (&fr)[GC], Real (&rad)[GC]) const
+    {
+        const double tbound = w.colscal[(size_t)in.ncol + col];
+        const Real semiss = (Real)in.emis[(size_t)(BAND - 1) * in.ncol + col];
+        // surface Planck (rrtmg_lw_setcoef.f90:190-194), FP64
+        const int i = clampi((int)(tbound - 159.0), 1, 180);
+        const double f = tbound - 159.0 - (double)i;
+        const Real plankbnd =
+            (Real)((double)semiss * ((double)plk[i - 1] + f * ((double)plk[i] - (double)plk[i - 1])));
+#pragma unroll
+        for (int j = 0; j < GC; ++j) rad[j] = fma(fr[j], plankbnd, ((Real)1 - semiss) * rad[j]);
+    }
+    // band sum of the radiances at level lev (up: 1, down: 0)
+    __device__ __forceinline__ void store(const Real (&rad)[GC], int lev, int up) const
+    {
+        Real *bf = (Real *)w.bflux + (size_t)(2 * (BAND - 1) + 1 - up) * (in.nlay + 1) * in.ncol;
+        const Real s = band_sum<BAND>(rad, g0);
+        if (first) at32(bf, (unsigned)(lev * in.ncol + col)) = s;
+    }
+};
+
+template <int GC, typename Real>
+struct alignas(GC * sizeof(Real) > 16 ? 16 : GC * sizeof(Real)) GVec {
+    Real x[GC];
+};
+
+// One unit by one wave (rrtmg_lw_rtrnmr.f90:483-716, clear sky): the downward
+// sweep keeps each layer's optical depths in the wave's scratch row,
+// [nlay][64][GC], for the upward one, which forms the sources again from them.
+// (Keeping transmittance and source instead doubles the traffic of the rows,
+// which leaves the caches: 1.27 ms against 1.14 at 32768 x 40.)
+template <int BAND, typename Real>
+__device__ __forceinline__ void lw_band_body(const LwUnit<BAND, Real> u, int lane, Real *__restrict__ row)
+{
+    constexpr int GC = LwUnit<BAND, Real>::GC;
+    using Vec = GVec<GC, Real>;
+    const int nlay = u.in.nlay;
+    Real rad[GC], fr[GC];
+    LwLayer<Real> c;
+#pragma unroll
+    for (int j = 0; j < GC; ++j) rad[j] = (Real)0;
+    u.store(rad, nlay, 0);  // drad(nlayers) stays 0
+    for (int lev = nlay; lev >= 1; --lev) {
+        u.load(c, lev);
+        Vec od;
+        u.depths(c, lev, od.x);
+        at32((Vec *)row, (unsigned)((lev - 1) * 64 + lane)) = od;
+        u.fracs(c, lev, fr);
+        const Real blay = u.planklay(c), dplankdn = u.planklev(lev - 1) - blay;
+#pragma unroll
+        for (int j = 0; j < GC; ++j) {
+            Real atr, tf;
+            u.transmit(od.x[j], atr, tf);
+            const Real bbd = fr[j] * fma(tf, dplankdn, blay);
+            rad[j] = fma(bbd - rad[j], atr, rad[j]);
+        }
+        u.store(rad, lev - 1, 0);
+    }
+    u.surface(fr, rad);
+    u.store(rad, 0, 1);
+    // the optical depths are read two levels ahead
+    Vec n1 = at32((const Vec *)row, (unsigned)lane), n2 = at32((const Vec *)row, (unsigned)(64 + lane));
     for (int lev = 1; lev <= nlay; ++lev) {
-        const Real bbugas = b0, atrans = a0;
-        b0 = b1;
-        b1 = b2;
-        b2 = b3;
-        b3 = at(s_bbu, lev + 3);
-        a0 = a1;
-        a1 = a2;
-        a2 = a3;
-        a3 = at(s_atr, lev + 3);
-        radlu = radlu + (bbugas - radlu) * atrans;
-        Real s = gsum.sum(active ? radlu : (Real)0, s_red);
-        if (active && g == 0) at32(bf_up, (unsigned)(lev * ncol + col)) = s;
+        const Vec od = n1;
+        n1 = n2;
+        if (lev + 1 < nlay) n2 = at32((const Vec *)row, (unsigned)((lev + 1) * 64 + lane));
+        u.load(c, lev);
+        u.fracs(c, lev, fr);
+        const Real blay = u.planklay(c), dplankup = u.planklev(lev) - blay;
+#pragma unroll
+        for (int j = 0; j < GC; ++j) {
+            Real atr, tf;
+            u.transmit(od.x[j], atr, tf);
+            const Real bbu = fr[j] * fma(tf, dplankup, blay);
+            rad[j] = fma(bbu - rad[j], atr, rad[j]);
+        }
+        u.store(rad, lev, 1);
     }
 }
 
-template <typename Real>
-__global__ __launch_bounds__(64) void lw_band_kernel(ColumnInputs in, LwWork w, const LwBand *__restrict__ bands,
-                                                     int nwaves, int blk0, int nblocks, int exp_off, int tfn_off,
-                                                     int plk_off, const Real *__restrict__ tab,
-                                                     const LwConst *__restrict__ cst, const WaveUnit *__restrict__ units)
+// One unit by a workgroup of LW_LWAVES waves, for calls too small to fill the
+// chip with waves: the layers' optics, which do not depend on each other, are
+// shared out among the waves (a layer takes some 4000 cycles of dependent loads
+// whoever computes it), then one wave sweeps down and the next up through the
+// stored transmittances and sources, leaving the radiances, and all form the
+// sums.  row: the workgroup's scratch, [nlay][4][64][GC] (transmittance, downward
+// source, upward source and then radiance, downward radiance) and one more [64][GC] (Planck fractions of the lowest layer).
+template <int WAVES, int BAND, typename Real>
+__device__ __forceinline__ void lw_band_layers(const LwUnit<BAND, Real> u, int wave, int lane, Real *__restrict__ row)
 {
-    extern __shared__ unsigned char smem_raw[];
-    Real *smem = (Real *)smem_raw;
-    const int blk = xcd_block();
-    if (blk >= nblocks) return;
-    const int tile = (blk0 + blk) / nwaves;
-    const WaveUnit u = units[(blk0 + blk) % nwaves];
-    const LwBand B = bands[u.band];
-    Real *s_bbu = (Real *)w.dstate + (size_t)blk * in.nlay * 64;
-    Real *s_atr = smem, *s_red = smem + (size_t)in.nlay * 64;
-#define BODY(b)                                                                                               \
-    case b - 1:                                                                                               \
-        lw_band_body<b, Real>(in, w, B, tab, tab, exp_off, tfn_off, plk_off, cst, u, tile, (int)threadIdx.x, s_atr, \
-                              s_bbu, s_red);                                                                  \
-        break;
-    switch (u.band) {
-        BODY(1) BODY(2) BODY(3) BODY(4) BODY(5) BODY(6) BODY(7) BODY(8)
-        BODY(9) BODY(10) BODY(11) BODY(12) BODY(13) BODY(14) BODY(15) BODY(16)
+    constexpr int GC = LwUnit<BAND, Real>::GC;
+    using Vec = GVec<GC, Real>;
+    const int nlay = u.in.nlay;
+    auto at = [&](int lev, int k) -> Vec & { return at32((Vec *)row, (unsigned)(((lev - 1) * 4 + k) * 64 + lane)); };
+    for (int lev = nlay - wave; lev >= 1; lev -= WAVES) {
+        LwLayer<Real> c;
+        u.load(c, lev);
+        Real od[GC], fr[GC];
+        u.depths(c, lev, od);
+        u.fracs(c, lev, fr);
+        const Real blay = u.planklay(c), dn = u.planklev(lev - 1) - blay, up = u.planklev(lev) - blay;
+        Vec atr, bbd, bbu, f;
+#pragma unroll
+        for (int j = 0; j < GC; ++j) {
+            Real tf;
+            u.transmit(od[j], atr.x[j], tf);
+            bbd.x[j] = fr[j] * fma(tf, dn, blay);
+            bbu.x[j] = fr[j] * fma(tf, up, blay);
+            f.x[j] = fr[j];
+        }
+        at(lev, 0) = atr;
+        at(lev, 1) = bbd;
+        at(lev, 2) = bbu;
+        if (lev == 1) at(nlay + 1, 0) = f;
     }
-#undef BODY
+    __syncthreads();
+    // sweep through the sources k, read four layers ahead; the radiances go to
+    // the places `to` (none if negative)
+    auto sweep = [&](Real (&rad)[GC], int first, int step, int k, int to) {
+        Vec a[4], b[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int lev = clampi(first + i * step, 1, nlay);
+            a[i] = at(lev, 0);
+            b[i] = at(lev, k);
+        }
+        for (int n = 0; n < nlay; n += 4)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (n + i >= nlay) break;
+                const int lev = first + (n + i) * step, next = clampi(lev + 4 * step, 1, nlay);
+                Vec r;
+#pragma unroll
+                for (int j = 0; j < GC; ++j) r.x[j] = rad[j] = fma(b[i].x[j] - rad[j], a[i].x[j], rad[j]);
+                a[i] = at(next, 0);
+                b[i] = at(next, k);
+                if (to >= 0) at(lev, to) = r;
+            }
+    };
+    // wave 0 down, wave 1 up; the latter needs the downward radiance at the
+    // surface where the surface reflects, and keeps no level of its own way down
+    Real rad[GC];
+#pragma unroll
+    for (int j = 0; j < GC; ++j) rad[j] = (Real)0;
+    if (wave == 0) {
+        u.store(rad, nlay, 0);
+        sweep(rad, nlay, -1, 1, 3);
+    } else if (wave == 1) {
+        sweep(rad, nlay, -1, 1, -1);
+        const Vec f = at(nlay + 1, 0);
+        u.surface(f.x, rad);
+        u.store(rad, 0, 1);
+        sweep(rad, 1, 1, 2, 2);
+    }
+    __syncthreads();
+    for (int lev = 1 + wave; lev <= nlay; lev += WAVES) {
+        u.store(at(lev, 3).x, lev - 1, 0);
+        u.store(at(lev, 2).x, lev, 1);
+    }
 }
 
-// FP32 band kernel with the band's k-tables in LDS.  Persistent workgroups of
-// LW_WGW waves claim work items from a global counter (next_item);
-// item = (group of LW_WGW tiles, unit r of a tile's unit list) covers the
-// group's LW_WGW x upt units of the band of unit r, one per wave.  Before an
-// item of another band the workgroup copies that band's k-tables (at most
-// plan.lds_bytes) into LDS; gathers from them then take LDS latency instead
-// of the L2 latency of 64-lane gathers that miss the 32 KB L1.  The
-// transmittance and upward source of each wave go to its global scratch row
-// (2 x nlay x 64; rows = waves of the grid, so they stay in the last-level
-// cache).
-template <typename Real>
-__global__ __launch_bounds__(64 * LW_WGW) void lw_band_lds_kernel(ColumnInputs in, LwWork w,
-                                                                  const LwBand *__restrict__ bands, LwLdsPlan plan,
-                                                                  int nwaves, int nitems, int exp_off, int tfn_off,
-                                                                  int plk_off, const Real *__restrict__ tab,
-                                                                  const LwConst *__restrict__ cst,
-                                                                  const WaveUnit *__restrict__ units)
+// Persistent workgroups of WAVES waves; work items (a band of CPW columns) from
+// a global counter, band by band, the bands with most work first.  LAYERS: a
+// workgroup takes an item (lw_band_layers), the (exp, tfn) pairs are read from
+// L2; else each wave takes items of its own, with the pairs in LDS.
+template <typename Real, int WAVES, bool LAYERS>
+__global__ __launch_bounds__(64 * WAVES)
+    __attribute__((amdgpu_waves_per_eu(2))) void lw_band_kernel(ColumnInputs in, LwWork w,
+                                                                const LwBand *__restrict__ bands, size_t row_elems,
+                                                                int et_off, int plk_off,
+                                                                const Real *__restrict__ tab,
+                                                                const LwConst *__restrict__ cst)
 {
-    static_assert(sizeof(Real) == 4, "FP32 only: the FP64 g-sum synchronises the workgroup");
-    extern __shared__ unsigned char smem_raw[];
-    Real *ktab = (Real *)smem_raw;
-    const int nlay = in.nlay;
-    const int ntiles = (in.ncol + TILE_COLS - 1) / TILE_COLS;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
-    Real *s_atr = (Real *)w.dstate + ((size_t)blockIdx.x * LW_WGW + wave) * 2 * nlay * 64;
-    Real *s_bbu = s_atr + (size_t)nlay * 64;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ int s_item;
-    int loaded = -1;
+    const ExpTfn<Real> *et;
+    if constexpr (LAYERS) {
+        et = (const ExpTfn<Real> *)(tab + et_off);
+    } else {
+        if (et_off >= 0) {
+            const uint4 *src = (const uint4 *)(tab + et_off);
+            constexpr int n = (int)((2 * (NTBL + 1) * sizeof(Real) + 15) / 16);
+            for (int i = threadIdx.x; i < n; i += 64 * WAVES) ((uint4 *)smem_raw)[i] = src[i];
+        }
+        __syncthreads();
+        et = (const ExpTfn<Real> *)smem_raw;
+    }
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+    Real *row = (Real *)w.dstate + ((size_t)blockIdx.x * (LAYERS ? 1 : WAVES) + (LAYERS ? 0 : wave)) * row_elems;
     for (;;) {
-        const int item = next_item(w.items, &s_item);
-        if (item >= nitems) break;
-        const int group = item / nwaves, r = item - group * nwaves;
-        const int b = units[r].band;
+        int item = 0;
+        if constexpr (LAYERS) {
+            item = __builtin_amdgcn_readfirstlane(next_item(w.items, &s_item));
+        } else {
+            if (lane == 0) item = atomicAdd(w.items, 1);
+            item = __builtin_amdgcn_readfirstlane(item);
+        }
+        // the item's band and its first column
+#define UNIT(b, e) LwUnit<b, Real>(in, w, bands[b - 1], tab, tab, tab, e, plk_off, cst, item * lw_cpw(b), in.ncol, lane)
+#define BODY(b)                                                                                                  \
+    {                                                                                                            \
+        const int n = (in.ncol + lw_cpw(b) - 1) / lw_cpw(b);                                                     \
+        if (item < n) {                                                                                          \
+            if constexpr (LAYERS)                                                                                \
+                lw_band_layers<WAVES>(UNIT(b, et), wave, lane, row);                                                  \
+            else if (sizeof(Real) == 4 || et_off >= 0)                                                           \
+                lw_band_body(UNIT(b, et), lane, row);                                                            \
+            else if constexpr (sizeof(Real) == 8)                                                                \
+                lw_band_body(UNIT(b, nullptr), lane, row);                                                       \
+            continue;                                                                                            \
+        }                                                                                                        \
+        item -= n;                                                                                               \
+    }
+        BODY(5) BODY(3) BODY(4) BODY(7) BODY(9) BODY(13) BODY(12) BODY(8)
+        BODY(1) BODY(6) BODY(15) BODY(16) BODY(11) BODY(2) BODY(10) BODY(14)
+#undef BODY
+#undef UNIT
+        return;
+    }
+}
+
+#pragma clang fp contract(fast)
+
+__constant__ constexpr LwTileSlots LW_TILE_SLOTS{};
+
+// FP32 kernel of the large calls: persistent 16-wave workgroups, one per CU,
+// with the (exp, tfn) pairs and one band's k-tables in LDS (absb of bands 3-5,
+// 75 KB, stays global).  Work item = one band of a tile of LW_TILE columns
+// (LwTileSlots), one unit of CPW columns per wave.  Each XCD claims the tiles
+// t = xcd (mod 8) from its own counter, so the bands that read a tile's
+// coefficients share an L2, and takes other XCDs' items when its own are gone.
+__global__ __launch_bounds__(1024) void lw_band_lds_kernel(ColumnInputs in, LwWork w,
+                                                           const LwBand *__restrict__ bands_lds, LwLdsPlan plan,
+                                                           size_t row_elems, int et_off, int plk_off,
+                                                           const float *__restrict__ tab,
+                                                           const LwConst *__restrict__ cst)
+{
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    constexpr int ET16 = (int)((2 * (NTBL + 1) * sizeof(float) + 15) / 16);
+    ExpTfn<float> *et = (ExpTfn<float> *)smem_raw;
+    float *ktab = (float *)(smem_raw + ET16 * 16);
+    for (int i = threadIdx.x; i < ET16; i += 1024) ((uint4 *)smem_raw)[i] = ((const uint4 *)(tab + et_off))[i];
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+    float *row = (float *)w.dstate + ((size_t)blockIdx.x * 16 + wave) * row_elems;
+    const int ntiles = (in.ncol + LW_TILE - 1) / LW_TILE;
+    __shared__ int s_item;
+    int loaded = -1, queue = 0;
+    for (;;) {
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            int it = -1;
+            for (; queue < 8; ++queue) {
+                const int x = ((int)blockIdx.x + queue) & 7;
+                const int n = ((ntiles - x + 7) >> 3) * LW_TILE_ITEMS;
+                const int k = n > 0 ? atomicAdd(w.items + x, 1) : n;
+                if (k < n) {
+                    it = (x + 8 * (k / LW_TILE_ITEMS)) * LW_TILE_ITEMS + k % LW_TILE_ITEMS;
+                    break;
+                }
+            }
+            s_item = it;
+        }
+        __syncthreads();
+        const int item = __builtin_amdgcn_readfirstlane(s_item);
+        if (item < 0) return;
+        const int tile = item / LW_TILE_ITEMS, k = item - tile * LW_TILE_ITEMS;
+        const LwTileSlot slot = LW_TILE_SLOTS.s[k];
+        const int b = slot.band - 1;
         if (b != loaded) {
-            const int t0 = plan.tab0[b], n = plan.tab0[b + 1] - t0;
-#pragma unroll 8
-            for (int i = threadIdx.x; i < n; i += 64 * LW_WGW) ktab[i] = tab[t0 + i];
+            // the band's k-tables but for [cut0, cut1), absb where it stays global
+            const int t0 = plan.tab0[b], n = plan.tab0[b + 1] - t0, c0 = plan.cut0[b], c1 = plan.cut1[b];
+            for (int i = threadIdx.x; i < n / 4; i += 1024)
+                if (i < c0 / 4 || i >= c1 / 4)
+                    ((float4 *)ktab)[i < c0 / 4 ? i : i - (c1 - c0) / 4] = ((const float4 *)(tab + t0))[i];
             __syncthreads();
             loaded = b;
         }
-        const int k = (r - plan.ubeg[b]) * LW_WGW + wave;
-        const int tile = group * LW_WGW + k / plan.upt[b];
-        if (tile >= ntiles) continue;
-        const WaveUnit u = units[plan.ubeg[b] + k % plan.upt[b]];
-        const LwBand B = bands[b];
-#define BODY(bb)                                                                                              \
-    case bb - 1:                                                                                              \
-        lw_band_body<bb, Real>(in, w, B, ktab, tab, exp_off, tfn_off, plk_off, cst, u, tile, lane, s_atr, s_bbu, \
-                               nullptr);                                                                      \
+        const int c0 = tile * LW_TILE + (slot.part * 16 + wave) * slot.cpw, cend = min((tile + 1) * LW_TILE, in.ncol);
+        if (c0 >= cend) continue;
+#define BODY(bb)                                                                                                  \
+    case bb - 1:                                                                                                  \
+        lw_band_body(LwUnit<bb, float>(in, w, bands_lds[bb - 1], ktab, bb >= 3 && bb <= 5 ? tab : ktab, tab, et,   \
+                                       plk_off, cst, c0, cend, lane),                                             \
+                     lane, row);                                                                                  \
         break;
         switch (b) {
             BODY(1) BODY(2) BODY(3) BODY(4) BODY(5) BODY(6) BODY(7) BODY(8)
@@ -448,31 +678,26 @@ static hipError_t launch_lw_t(const ColumnInputs &in, const LwOutputs &out, cons
     if (ev) (void)hipEventRecord(ev[0], s);
     hipLaunchKernelGGL(lw_prep_kernel<Real>, dim3(nbl), dim3(256), 0, s, in, w, t.cst);
     hipLaunchKernelGGL(lw_column_kernel, dim3(nb), dim3(256), 0, s, in, w);
-    const int ntiles = (in.ncol + TILE_COLS - 1) / TILE_COLS;
-    const size_t shmem = lw_fwd_lds_bytes(in.nlay, sizeof(Real));
     if (ev) (void)hipEventRecord(ev[1], s);
-    const int nblocks = ntiles * t.desc.nwaves;
+    hipLaunchKernelGGL(reset_items_kernel, dim3(1), dim3(8), 0, s, w.items);
+    const size_t row = lw_fwd_state_bytes(in.nlay, 1), et = (2 * (NTBL + 1) * sizeof(Real) + 15) / 16 * 16;
+    const int et_off = smooth ? -1 : t.desc.et_tbl;
     if constexpr (sizeof(Real) == 4) {
-        if (t.lds && !smooth) {
-            const int nitems = (ntiles + LW_WGW - 1) / LW_WGW * t.desc.nwaves;
-            hipLaunchKernelGGL(reset_items_kernel, dim3(1), dim3(1), 0, s, w.items);
-            hipLaunchKernelGGL(lw_band_lds_kernel<Real>, dim3(lw_lds_grid(t.plan, in.ncol, t.desc.nwaves)),
-                               dim3(64 * LW_WGW), (size_t)t.plan.lds_bytes, s, in, w, t.bands_lds, t.plan,
-                               t.desc.nwaves, nitems, t.desc.exp_tbl, t.desc.tfn_tbl, t.desc.totplnk,
-                               (const Real *)t.tab, t.cst, t.units);
-            if (ev) (void)hipEventRecord(ev[2], s);
-            hipLaunchKernelGGL(lw_finish_kernel<Real>, dim3(nbl), dim3(256), 0, s, in, w, out, t.bands, heatfac);
-            if (ev) (void)hipEventRecord(ev[3], s);
-            return hipGetLastError();
-        }
+        if (w.kind == 16)
+            hipLaunchKernelGGL(lw_band_lds_kernel, dim3(w.chunk), dim3(1024), (size_t)t.plan.fwd_lds_bytes, s, in, w,
+                               t.bands_fwd, t.plan, row, et_off, t.desc.totplnk, (const float *)t.tab, t.cst);
     }
-    // launches of at most w.chunk wave units, each reusing the scratch rows
-    for (int b0 = 0; b0 < nblocks; b0 += w.chunk) {
-        const int nb_c = std::min(w.chunk, nblocks - b0);
-        hipLaunchKernelGGL(lw_band_kernel<Real>, dim3(xcd_grid(nb_c)), dim3(64), shmem, s, in, w, t.bands,
-                           t.desc.nwaves, b0, nb_c, smooth ? -1 : t.desc.exp_tbl, smooth ? -1 : t.desc.tfn_tbl,
-                           t.desc.totplnk, (const Real *)t.tab, t.cst, t.units);
+    if constexpr (sizeof(Real) == 8) {
+        if (w.kind == 8)
+            hipLaunchKernelGGL((lw_band_kernel<Real, 8, false>), dim3(w.chunk), dim3(512), smooth ? 0 : et, s, in, w,
+                               t.bands, row, et_off, t.desc.totplnk, (const Real *)t.tab, t.cst);
     }
+    if (w.kind == 1)
+        hipLaunchKernelGGL((lw_band_kernel<Real, 8, true>), dim3(w.chunk), dim3(512), 0, s, in, w, t.bands,
+                           lw_fwd_layers_bytes(in.nlay, 1), et_off, t.desc.totplnk, (const Real *)t.tab, t.cst);
+    if (w.kind == 2)
+        hipLaunchKernelGGL((lw_band_kernel<Real, 4, true>), dim3(w.chunk), dim3(256), 0, s, in, w, t.bands,
+                           lw_fwd_layers_bytes(in.nlay, 1), et_off, t.desc.totplnk, (const Real *)t.tab, t.cst);
     if (ev) (void)hipEventRecord(ev[2], s);
     hipLaunchKernelGGL(lw_finish_kernel<Real>, dim3(nbl), dim3(256), 0, s, in, w, out, t.bands, heatfac);
     if (ev) (void)hipEventRecord(ev[3], s);

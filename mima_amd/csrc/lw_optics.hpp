@@ -8,6 +8,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "dual.hpp"
 #include "rrtmg_device.hpp"
 #include "rrtmg_types.hpp"
@@ -24,15 +26,28 @@ struct LwLayer {
     int jp, jt, jt1, inds, indf, indm, indlay;
 };
 
+// a lane's byte offset within a group's columns: 32 bits in FP32 (16 bytes
+// times a column count that check_common bounds), 64 in FP64
+template <typename Real>
+using LaneOffset = typename std::conditional<sizeof(Real) == 4, unsigned, size_t>::type;
+
 template <typename Real>
 __device__ __forceinline__ void lw_load_layer(LwLayer<Real> &c, const Real *__restrict__ coef,
                                               const int *__restrict__ ipk, int lay, int col, int ncol, int nlay)
 {
     const unsigned ix = (unsigned)(lay * ncol + col);
-    // the (layer, column) record, [lay][col][LWF_STRIDE], 16-byte aligned
-    const Real *rec = (const Real *)__builtin_assume_aligned(coef + (size_t)ix * LWF_STRIDE, 16);
+    // the layer's groups of four fields, [group][col][4]; groups whose fields
+    // the caller does not use are not loaded
+    struct alignas(16) Group {
+        Real x[4];
+    };
+    const Group *base = (const Group *)coef + (size_t)lay * LWF_GROUPS * ncol;
+    Group g[LWF_GROUPS];
+#pragma unroll
+    for (int k = 0; k < LWF_GROUPS; ++k)
+        g[k] = *(const Group *)((const char *)(base + (size_t)k * ncol) + (LaneOffset<Real>)col * sizeof(Group));
     (void)nlay;
-#define LD(f, F) c.f = rec[F]
+#define LD(f, F) c.f = g[(F) / 4].x[(F) % 4]
     LD(fac00, LWF_FAC00); LD(fac01, LWF_FAC01); LD(fac10, LWF_FAC10); LD(fac11, LWF_FAC11);
     LD(colh2o, LWF_COLH2O); LD(colco2, LWF_COLCO2); LD(colo3, LWF_COLO3); LD(coln2o, LWF_COLN2O);
     LD(colco, LWF_COLCO); LD(colch4, LWF_COLCH4); LD(colo2, LWF_COLO2); LD(colbrd, LWF_COLBRD);
@@ -74,6 +89,7 @@ struct Eta {
 template <typename V, typename S>
 __device__ __forceinline__ Eta<V> lw_eta(V cola, V colb, S rat, S mult)
 {
+#pragma clang fp contract(off)  // the same bits in every kernel (lw_rows.hpp)
     Eta<V> e;
     e.speccomb = cola + rat * colb;
     e.specparm = fdiv(cola, e.speccomb);
@@ -155,6 +171,7 @@ __device__ __forceinline__ V lw_pfrac(const LTab<Real> &T, int off, const Eta<V>
 template <typename V, typename S>
 __device__ __forceinline__ V lw_adjcol(V col, V coldry, S chiref, S thresh, S base, S ex)
 {
+#pragma clang fp contract(off)
     V rat = fdiv((S)1.e20 * fdiv(col, coldry), chiref);
     if (rat > thresh) return (base + pow(rat - base, ex)) * chiref * coldry * (S)1.e-20;
     return col;

@@ -86,7 +86,7 @@ using gptr = __attribute__((address_space(1))) T *;
 template <typename T>
 using lptr = __attribute__((address_space(3))) T *;
 
-[[maybe_unused]] static __global__ void reset_items_kernel(int *items) { *items = 0; }
+[[maybe_unused]] static __global__ void reset_items_kernel(int *items) { items[threadIdx.x] = 0; }
 
 // Next work item of a persistent workgroup, claimed from a global counter
 // (dynamic balance: items differ in cost, e.g. night columns in SW); every

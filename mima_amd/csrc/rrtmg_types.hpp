@@ -76,6 +76,7 @@ struct LwBand {
 struct LwTables {
     LwBand band[16];
     int exp_tbl, tfn_tbl;     // 10001 entries each
+    int et_tbl;               // the same as 10001 (exp, tfn) pairs
     int totplnk;              // [band][181]
     int nwaves;
 };
@@ -96,6 +97,41 @@ constexpr int sw_ng(int jb)
          : jb == 22 ? 2 : jb == 23 ? 10 : jb == 24 ? 8 : jb == 25 ? 6 : jb == 26 ? 6 : jb == 27 ? 8
          : jb == 28 ? 6 : 12;
 }
+
+// Work of one lane: GC consecutive g-points of one column and band; LPC
+// adjacent lanes cover the band, CPW columns a wave.  The last lane of a band
+// whose g-points are not a multiple of GC holds dummies past the band's end.
+template <int BAND>
+struct LwLanes {
+    static constexpr int NG = lw_ng(BAND), GC = NG >= 4 ? 4 : 2, LPC = (NG + GC - 1) / GC, CPW = 64 / LPC;
+};
+
+// The items of a tile of LW_TILE columns (a multiple of 21, and 16 units of 64
+// lanes but for a rest): each of 16 units of one band, the heavy bands first
+constexpr int LW_TILE = 1008;
+struct LwTileSlot {
+    unsigned char band, part, cpw;
+};
+constexpr int lw_cpw(int band) { return 64 / ((lw_ng(band) + 3) / 4); }
+constexpr int lw_tile_parts(int band) { return (LW_TILE + 16 * lw_cpw(band) - 1) / (16 * lw_cpw(band)); }
+constexpr int lw_tile_items()
+{
+    int n = 0;
+    for (int b = 1; b <= 16; ++b) n += lw_tile_parts(b);
+    return n;
+}
+constexpr int LW_TILE_ITEMS = lw_tile_items();
+struct LwTileSlots {
+    LwTileSlot s[LW_TILE_ITEMS];
+    constexpr LwTileSlots() : s()
+    {
+        constexpr int order[16] = {5, 3, 4, 7, 9, 13, 12, 8, 1, 6, 15, 16, 11, 2, 10, 14};
+        int n = 0;
+        for (int i = 0; i < 16; ++i)
+            for (int p = 0; p < lw_tile_parts(order[i]); ++p)
+                s[n++] = {(unsigned char)order[i], (unsigned char)p, (unsigned char)lw_cpw(order[i])};
+    }
+};
 
 // species-parameter counts of the k-tables per band, lower/upper atmosphere
 // (rrtmg_lw_init.f90:208-209, rrtmg_sw_init.f90:183-184); checked against
@@ -136,18 +172,22 @@ struct LwConst {
     float chi_ratio_f[LW_NCHI_RATIO];
 };
 
+// ordered so that a band that needs few of them needs few groups of four
 enum LwField {
     LWF_FAC00, LWF_FAC01, LWF_FAC10, LWF_FAC11,
-    LWF_COLH2O, LWF_COLCO2, LWF_COLO3, LWF_COLN2O, LWF_COLCO, LWF_COLCH4, LWF_COLO2, LWF_COLBRD,
-    LWF_SELFFAC, LWF_SELFFRAC, LWF_FORFAC, LWF_FORFRAC,
-    LWF_MINORFRAC, LWF_SCALEMINOR, LWF_SCALEMINORN2, LWF_COLDRY, LWF_PAVEL,
-    LWF_WX1, LWF_WX2, LWF_WX3, LWF_WX4, LWF_TLAYFRAC,
+    LWF_COLH2O, LWF_COLCO2, LWF_SELFFAC, LWF_SELFFRAC,
+    LWF_FORFAC, LWF_FORFRAC, LWF_MINORFRAC, LWF_TLAYFRAC,
+    LWF_COLO3, LWF_COLN2O, LWF_COLDRY, LWF_PAVEL,
+    LWF_COLCH4, LWF_COLO2, LWF_COLBRD, LWF_SCALEMINOR,
+    LWF_SCALEMINORN2, LWF_COLCO, LWF_WX1, LWF_WX2,
+    LWF_WX3, LWF_WX4,
     LWF_COUNT
 };
-// the forward prep's coefficient record of one (layer, column): LWF_COUNT
-// fields padded to a 16-byte multiple, so a band kernel lane loads its
-// column's fields with a few 16-byte loads
+// the forward prep's coefficients: groups of four fields, [lay][group][col][4],
+// so a lane loads its column's group with one 16-byte load beside its
+// neighbours', and a band only the groups it uses
 constexpr int LWF_STRIDE = (LWF_COUNT + 3) / 4 * 4;
+constexpr int LWF_GROUPS = LWF_STRIDE / 4;
 
 // The backward's coefficient records: per (layer, column) a value record of
 // LWF_STRIDE / SWF_STRIDE fields (the forward's record) and a derivative
@@ -159,8 +199,8 @@ constexpr int LWF_STRIDE = (LWF_COUNT + 3) / 4 * 4;
 // the latter also on T); selffac/forfac (stored times the water column) on T
 // and q.  The derivative record lists each field's components in field order,
 // d/dT before d/dq before d/dO3, padded to a 16-byte multiple.
-constexpr unsigned LW_DMASK[LWF_COUNT] = {1, 1, 1, 1, 2, 2, 6, 2, 2, 2, 2, 6, 3,
-                                          1, 3, 1, 1, 1, 7, 2, 0, 2, 2, 2, 2, 1};
+constexpr unsigned LW_DMASK[LWF_COUNT] = {1, 1, 1, 1, 2, 2, 3, 1, 3, 1, 1, 1, 6,
+                                          2, 2, 0, 2, 2, 6, 1, 7, 2, 2, 2, 2, 2};
 constexpr unsigned SW_DMASK[SWF_COUNT] = {1, 1, 1, 1, 2, 2, 6, 2, 2, 2, 3, 1, 3, 1};
 constexpr int dmask_count(unsigned m) { return (int)(m & 1u) + (int)((m >> 1) & 1u) + (int)((m >> 2) & 1u); }
 // offset of field f's first derivative in the derivative record

@@ -203,6 +203,7 @@ static std::vector<double> reduce(const TableFile &t, const std::string &name, b
 static int pack(std::vector<double> &buf, const std::vector<double> &red, int rows, int ng, bool gfirst)
 {
     if (red.empty()) return -1;
+    buf.resize((buf.size() + 3) / 4 * 4);  // rows of a multiple of four g-points load as aligned vectors
     int off = (int)buf.size();
     buf.resize(buf.size() + (size_t)rows * ng);
     for (int r = 0; r < rows; ++r)
@@ -215,6 +216,7 @@ static void exp_table(std::vector<double> &buf, int *off_exp, int *off_tfn)
 {
     // rrtmg_lw_init.f90:106-123 / rrtmg_sw_init.f90:94-104
     const double bpade = 1.0 / 0.278, expeps = 1.e-20;
+    buf.resize((buf.size() + 3) / 4 * 4);
     *off_exp = (int)buf.size();
     buf.resize(buf.size() + NTBL + 1);
     double *ex = &buf[*off_exp];
@@ -474,6 +476,12 @@ bool build_lw(const std::string &path, double cpdair, LwHost &h, std::string &er
     exp_table(buf, &h.tab.exp_tbl, &h.tab.tfn_tbl);
     h.tab.totplnk = (int)buf.size();
     buf.insert(buf.end(), totplnk.begin(), totplnk.end());  // already [band][181]
+    buf.resize((buf.size() + 3) / 4 * 4);
+    h.tab.et_tbl = (int)buf.size();
+    for (int i = 0; i <= NTBL; ++i) {
+        buf.push_back(buf[h.tab.exp_tbl + i]);
+        buf.push_back(buf[h.tab.tfn_tbl + i]);
+    }
     h.tab.nwaves = build_schedule(16, ngv, h.units);
     return true;
 }
