@@ -65,6 +65,7 @@ struct SideTables {
     WaveUnit *units = nullptr;
     double *preflog = nullptr, *tref = nullptr;  // SW
     LwConst *cst = nullptr;                      // LW
+    int ncu = 1;                                 // SW: compute units
     LwBand *bands_fwd = nullptr;                 // LW: the same for the forward kernel's copy
     LwBand *bands_lds = nullptr;                 // LW: offsets relative to each band's first k-table element
     LwLdsPlan plan{};                            // LW: schedule of the LDS-table kernel
@@ -376,6 +377,10 @@ int rrtmg_hip_sw_init(double cpdair, const char *table_dir)
         }
     }
     if (rc) return fail(rc, "uploading SW tables failed");
+    {
+        int lds = 0;
+        if (lds_device(&s->swd.ncu, &lds)) return fail(RRTMG_HIP_EDEVICE, "device attribute query failed");
+    }
     s->swd.cpdair = cpdair;
     s->swd.ready = true;
     // the no-allocation entry point's scratch address on this device; a
@@ -571,7 +576,6 @@ int sw_forward(int ncol, int nlay, int icld, int iaer, const double *play, const
     hipStream_t st = (hipStream_t)stream;
     const int mixed = g_prec == RRTMG_HIP_PREC_MIXED;
     const size_t rs = mixed ? sizeof(float) : sizeof(double);
-    if ((rc = check_lds(sw_fwd_lds_bytes(nlay, rs)))) return rc;
 
     // workspace: [input-check flag (fixed region only)] coefficient records,
     // packed indices, laytrop, laysolfr, band fluxes, scratch rows
@@ -582,25 +586,30 @@ int sw_forward(int ncol, int nlay, int icld, int iaer, const double *play, const
     const size_t o_lsf = off; off = align_up(off + sizeof(int) * 14 * ncol);
     const size_t o_bf = off; off = align_up(off + rs * 14 * 2 * n3);
     const size_t o_ds = off;
-    const int units = (ncol + TILE_COLS - 1) / TILE_COLS * s->sw.tab.nwaves;
-    const size_t unit_bytes = cl ? sw_cloud_row_bytes(nlay, rs) : sw_fwd_state_bytes(nlay, rs);
-    int chunk;
+    const int units = (ncol + TILE_COLS - 1) / TILE_COLS * s->sw.tab.nwaves;  // of the cloudy band kernel
+    const bool smooth = g_prec == RRTMG_HIP_PREC_FP64_SMOOTH;
+    int kind = sw_fwd_kind(ncol, s->swd.ncu, smooth), rows = 0, chunk = 0;
     char *wb;
     int *flag = nullptr;
     StreamWork *W = nullptr;
     if (fx) {
-        const size_t avail = fx->cap > 256 ? fx->cap - 256 : 0;
-        const size_t rows = avail > o_ds ? (avail - o_ds) / unit_bytes : 0;
-        if (rows < (size_t)std::min(units, 8))
+        // one wave's row is enough; the rest of the region is for more
+        kind = SW_WAVE2;
+        const size_t avail = fx->cap > 512 ? fx->cap - 512 : 0;
+        rows = avail > o_ds ? sw_fwd_rows(ncol, nlay, rs, s->swd.ncu, kind, avail - o_ds) : 0;
+        if (rows < 1)
             return fail(RRTMG_HIP_EINVAL, "ncol x nlay too large for the no-allocation entry point (needs more than " +
-                                              std::to_string(o_ds + 8 * unit_bytes + 256) + " bytes of its " +
-                                              std::to_string(fx->cap) + "-byte scratch array); call rrtmg_hip_sw");
-        chunk = (int)std::min((size_t)units, rows);
+                                              std::to_string(o_ds + sw_fwd_rows_bytes(nlay, rs, kind) + 512) +
+                                              " bytes of its " + std::to_string(fx->cap) +
+                                              "-byte scratch array); call rrtmg_hip_sw");
         flag = (int *)fx->p;
-        wb = (char *)fx->p + 256;
+        wb = (char *)fx->p + 512;
     } else {
         W = &s->work(st);
-        chunk = vjp_chunk(units, unit_bytes);
+        if (cl)
+            chunk = vjp_chunk(units, sw_cloud_row_bytes(nlay, rs));
+        else
+            rows = std::max(1, sw_fwd_rows(ncol, nlay, rs, s->swd.ncu, kind, VJP_SCRATCH_BYTES));
     }
     if (ptr_kind == RRTMG_HIP_DEVICE && g_checks) {
         std::vector<NamedArray> a;
@@ -631,7 +640,9 @@ int sw_forward(int ncol, int nlay, int icld, int iaer, const double *play, const
             return rc;
     }
     int ck = 0;
-    off = align_up(o_ds + (size_t)chunk * unit_bytes);
+    off = align_up(o_ds + (cl ? chunk * sw_cloud_row_bytes(nlay, rs) : rows * sw_fwd_rows_bytes(nlay, rs, kind)));
+    const size_t o_it = off; if (!fx) off = align_up(off + 2 * sizeof(int));
+    const size_t o_day = off; if (!fx && !cl) off = align_up(off + sizeof(int) * ncol);
     // cloud path: flags, four-stream band fluxes, partial-cloud count
     const size_t o_cfl = off; if (cl) off = align_up(off + sizeof(int) * n2);
     const size_t o_cbf = off; if (cl) off = align_up(off + rs * 14 * 4 * n3);
@@ -655,7 +666,10 @@ int sw_forward(int ncol, int nlay, int icld, int iaer, const double *play, const
     w.laysolfr = (int *)(wb + o_lsf);
     w.bflux = wb + o_bf;
     w.dstate = wb + o_ds;
-    w.chunk = chunk;
+    w.rows = rows;
+    w.kind = kind;
+    w.items = fx ? (int *)((char *)fx->p + 256) : (int *)(wb + o_it);
+    w.day = fx || cl ? nullptr : (int *)(wb + o_day);
     SwCloudWork cw;
     SwClouds cld{};
     if (cl) {

@@ -38,8 +38,11 @@ struct SwWork {
     int *laytrop = nullptr;   // [ncol]
     int *laysolfr = nullptr;  // [14][ncol]
     void *bflux = nullptr;    // [14][2][nlay+1][ncol] of Real
-    void *dstate = nullptr;   // [chunk][nlay+1][64] of Real: prupd of each wave of a band-kernel launch
-    int chunk = 0;            // wave units per band-kernel launch (rows of dstate)
+    void *dstate = nullptr;   // [rows] scratch rows, sw_fwd_rows_bytes each
+    int rows = 0;
+    int kind = 0;             // which band kernel (sw_fwd_kind)
+    int *items = nullptr;     // work-item counter of the band kernel, number of day columns
+    int *day = nullptr;       // [ncol] the day columns, or NULL: the band kernel takes every column
 };
 struct LwWork {
     void *coef = nullptr;     // [nlay][ncol][LWF_STRIDE] of Real (one record per layer and column)
@@ -320,7 +323,43 @@ inline int vjp_chunk(int units, size_t bytes_per_unit)
     if (c < 8) c = 8;
     return units < (int)c ? units : (int)c;
 }
-inline size_t sw_fwd_state_bytes(int nlay, size_t real_size) { return real_size * 2 * (size_t)(nlay + 1) * 64; }
+// the SW forward kernel: a wave per unit with four or two g-points a lane, or a
+// workgroup of eight or four waves per unit, two g-points a lane
+enum SwKind { SW_WAVE4, SW_WAVE2, SW_GROUP8, SW_GROUP4 };
+// units of work of the SW forward: CPW columns of a band
+inline size_t sw_fwd_units(int ncol, int kind)
+{
+    size_t n = 0;
+    for (int b = 16; b <= 29; ++b) {
+        const int cpw = sw_cpw(b, kind == SW_WAVE4 ? 4 : 2);
+        n += ((size_t)ncol + cpw - 1) / cpw;
+    }
+    return n;
+}
+// Half of a model's columns are day.  Workgroups of eight waves where they do
+// not fill the chip twice over (512 x 40: 44 us, 68 with four); of four up to
+// where waves of their own do as well (4096 x 40: 238 us, 291; 8192 x 40: 429,
+// 348); four g-points a lane where that many lanes fill it too (8192 x 40: 376
+// us, 348 with two; 12000 x 40: 429, 534).  FP64's lines lie there as well.
+inline int sw_fwd_kind(int ncol, int ncu, bool smooth)
+{
+    if (!smooth && sw_fwd_units(ncol, SW_GROUP8) <= 2 * (size_t)ncu) return SW_GROUP8;
+    if (!smooth && ncol < 6144) return SW_GROUP4;
+    return ncol < 10240 ? SW_WAVE2 : SW_WAVE4;
+}
+// a scratch row: of a wave, or of a workgroup
+inline size_t sw_fwd_rows_bytes(int nlay, size_t real_size, int kind)
+{
+    const size_t vals = kind == SW_WAVE4 ? 4 * 2 : kind == SW_WAVE2 ? 2 * 2 : 2 * 10;
+    return real_size * vals * (size_t)(nlay + 1) * 64;
+}
+// its rows: those of the workgroups that fit the chip at once, no more than
+// there is work for or than `bytes` hold
+inline int sw_fwd_rows(int ncol, int nlay, size_t real_size, int ncu, int kind, size_t bytes)
+{
+    const size_t fit = (size_t)ncu * (kind <= SW_WAVE2 ? (real_size == 4 ? 16 : 8) : kind == SW_GROUP8 ? 1 : 2);
+    return (int)std::min({bytes / sw_fwd_rows_bytes(nlay, real_size, kind), sw_fwd_units(ncol, kind), fit});
+}
 // LW forward: the optical depths of a lane's g-points, up to four
 inline size_t lw_fwd_state_bytes(int nlay, size_t real_size) { return real_size * 4 * (size_t)nlay * 64; }
 // and of its form that shares the layers of a unit among the waves of a
@@ -363,7 +402,6 @@ inline int lw_fwd_grid(int ncol, int nlay, size_t real_size, int ncu, int kind)
                                      : lw_fwd_units(ncol);
     return (int)std::max<size_t>(1, std::min({rows, items, (size_t)ncu * (kind == 2 ? 2 : 1)}));
 }
-inline size_t sw_fwd_lds_bytes(int, size_t real_size) { return real_size * 64; }
 __host__ __device__ inline size_t sw_vjp_state_bytes(int nlay, size_t real_size)
 {
     return real_size * (4 * (size_t)(nlay + 1) + 5 * (size_t)nlay) * 64;

@@ -357,11 +357,6 @@ struct LwUnit {
     }
 };
 
-template <int GC, typename Real>
-struct alignas(GC * sizeof(Real) > 16 ? 16 : GC * sizeof(Real)) GVec {
-    Real x[GC];
-};
-
 // One unit by one wave (rrtmg_lw_rtrnmr.f90:483-716, clear sky): the downward
 // sweep keeps each layer's optical depths in the wave's scratch row,
 // [nlay][64][GC], for the upward one, which forms the sources again from them.

@@ -8,8 +8,6 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#include <type_traits>
-
 #include "dual.hpp"
 #include "rrtmg_device.hpp"
 #include "rrtmg_types.hpp"
@@ -25,11 +23,6 @@ struct LwLayer {
     Real wx1, wx2, wx3, wx4, tlayfrac;
     int jp, jt, jt1, inds, indf, indm, indlay;
 };
-
-// a lane's byte offset within a group's columns: 32 bits in FP32 (16 bytes
-// times a column count that check_common bounds), 64 in FP64
-template <typename Real>
-using LaneOffset = typename std::conditional<sizeof(Real) == 4, unsigned, size_t>::type;
 
 template <typename Real>
 __device__ __forceinline__ void lw_load_layer(LwLayer<Real> &c, const Real *__restrict__ coef,

@@ -28,25 +28,6 @@ namespace rrtmg {
 // that the size of the call selects.
 #pragma clang fp contract(off)
 
-// GC consecutive values of a table row of NG g-points, from element offset e.
-// Tables start at multiples of four elements (tables.cpp), so four (two where
-// NG is not a multiple of four) values are one aligned load.
-template <int NG, int GC, typename Real>
-__device__ __forceinline__ void load_row(Real (&v)[GC], const Real *__restrict__ t, unsigned e)
-{
-    constexpr int W = NG % 4 == 0 && GC % 4 == 0 ? 4 : 2;
-    static_assert(GC % W == 0, "chunks of g-points are even");
-    struct alignas(W * sizeof(Real) > 16 ? 16 : W * sizeof(Real)) Vec {
-        Real x[W];
-    };
-#pragma unroll
-    for (int i = 0; i < GC; i += W) {
-        const Vec p = *(const Vec *)((const char *)t + (e + i) * (unsigned)sizeof(Real));
-#pragma unroll
-        for (int j = 0; j < W; ++j) v[i + j] = p.x[j];
-    }
-}
-
 // The three rows of the lower atmosphere's eta interpolation
 // (rrtmg_lw_taumol.f90:550-668) from one base row: below 0.125 the cubic
 // scheme on rows js, js+1, js+2, above 0.875 on js-1, js, js+1, between them

@@ -2,6 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 namespace rrtmg {
 
 __host__ __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
@@ -74,6 +76,36 @@ __device__ __forceinline__ const T &at32(const T *base, unsigned i)
 {
     return *(const T *)((const char *)base + i * (unsigned)sizeof(T));
 }
+
+// a lane's byte offset within a group's columns: 32 bits in FP32 (16 bytes
+// times a column count that check_common bounds), 64 in FP64
+template <typename Real>
+using LaneOffset = typename std::conditional<sizeof(Real) == 4, unsigned, size_t>::type;
+
+// GC consecutive values of a table row of NG g-points, from element offset e.
+// Tables start at multiples of four elements (tables.cpp), so four (two where
+// NG is not a multiple of four) values are one aligned load.
+template <int NG, int GC, typename Real>
+__device__ __forceinline__ void load_row(Real (&v)[GC], const Real *__restrict__ t, unsigned e)
+{
+    constexpr int W = NG % 4 == 0 && GC % 4 == 0 ? 4 : 2;
+    static_assert(GC % W == 0, "chunks of g-points are even");
+    struct alignas(W * sizeof(Real) > 16 ? 16 : W * sizeof(Real)) Vec {
+        Real x[W];
+    };
+#pragma unroll
+    for (int i = 0; i < GC; i += W) {
+        const Vec p = *(const Vec *)((const char *)t + (e + i) * (unsigned)sizeof(Real));
+#pragma unroll
+        for (int j = 0; j < W; ++j) v[i + j] = p.x[j];
+    }
+}
+
+// a lane's values of GC g-points in memory
+template <int GC, typename Real>
+struct alignas(GC * sizeof(Real) > 16 ? 16 : GC * sizeof(Real)) GVec {
+    Real x[GC];
+};
 
 // Zeroes the work-item counter of a persistent band kernel (a kernel, not a
 // memset, so that the sequence can be captured in a graph).

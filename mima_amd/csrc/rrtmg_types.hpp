@@ -56,9 +56,9 @@ enum SwField {
     SWF_SELFFAC, SWF_SELFFRAC, SWF_FORFAC, SWF_FORFRAC,
     SWF_COUNT
 };
-// the forward prep's coefficient record of one (layer, column), padded to a
-// 16-byte multiple (as LWF_STRIDE)
+// the forward prep's coefficients, in groups of four fields (as LWF_STRIDE)
 constexpr int SWF_STRIDE = (SWF_COUNT + 3) / 4 * 4;
+constexpr int SWF_GROUPS = SWF_STRIDE / 4;
 
 // ---------------------------------------------------------------------------
 // LW
@@ -105,6 +105,15 @@ template <int BAND>
 struct LwLanes {
     static constexpr int NG = lw_ng(BAND), GC = NG >= 4 ? 4 : 2, LPC = (NG + GC - 1) / GC, CPW = 64 / LPC;
 };
+
+// The same of a shortwave band: four g-points a lane (W = 4) where the band's
+// count is a multiple of four, two elsewhere and with W = 2, with no dummies: a
+// dummy's two-stream layer would cost as much as a g-point's.
+template <int JB, int W>
+struct SwLanes {
+    static constexpr int NG = sw_ng(JB), GC = W == 4 && NG % 4 == 0 ? 4 : 2, LPC = NG / GC, CPW = 64 / LPC;
+};
+constexpr int sw_cpw(int jb, int W) { return 64 / (sw_ng(jb) / (W == 4 && sw_ng(jb) % 4 == 0 ? 4 : 2)); }
 
 // The items of a tile of LW_TILE columns (a multiple of 21, and 16 units of 64
 // lanes but for a rest): each of 16 units of one band, the heavy bands first

@@ -45,6 +45,34 @@ __device__ __forceinline__ void sw_load_layer(SwLayer<Real> &c, const Real *__re
     c.indf = unpack_indf(w);
 }
 
+// the same from the groups of four fields, [lay][group][col][4]
+template <typename Real>
+__device__ __forceinline__ void sw_load_groups(SwLayer<Real> &c, const Real *__restrict__ coef,
+                                               const int *__restrict__ ipk, int lay, int col, int ncol)
+{
+    const unsigned ix = (unsigned)(lay * ncol + col);
+    struct alignas(16) Group {
+        Real x[4];
+    };
+    const Group *base = (const Group *)coef + (size_t)lay * SWF_GROUPS * ncol;
+    Group g[SWF_GROUPS];
+#pragma unroll
+    for (int k = 0; k < SWF_GROUPS; ++k)
+        g[k] = *(const Group *)((const char *)(base + (size_t)k * ncol) + (LaneOffset<Real>)col * sizeof(Group));
+#define LD(f, F) c.f = g[(F) / 4].x[(F) % 4]
+    LD(fac00, SWF_FAC00); LD(fac01, SWF_FAC01); LD(fac10, SWF_FAC10); LD(fac11, SWF_FAC11);
+    LD(colh2o, SWF_COLH2O); LD(colco2, SWF_COLCO2); LD(colo3, SWF_COLO3); LD(colch4, SWF_COLCH4);
+    LD(colo2, SWF_COLO2); LD(colmol, SWF_COLMOL);
+    LD(selffac, SWF_SELFFAC); LD(selffrac, SWF_SELFFRAC); LD(forfac, SWF_FORFAC); LD(forfrac, SWF_FORFRAC);
+#undef LD
+    int w = at32(ipk, ix);
+    c.jp = unpack_jp(w);
+    c.jt = unpack_jt(w);
+    c.jt1 = unpack_jt1(w);
+    c.inds = unpack_inds(w);
+    c.indf = unpack_indf(w);
+}
+
 // Per-column part of the SW prep for column col (after the per-layer part,
 // whose packed indices ipk hold jp): laytrop and the solar-source reference
 // layer of each band, laysolfr[b * ncol + col].  Bands searching the lower
@@ -107,6 +135,7 @@ struct Tab {
 template <typename R>
 __device__ __forceinline__ void sw_eta(R cola, R colb, R strrat, R mult, R &speccomb, int &js, R &fs)
 {
+#pragma clang fp contract(off)  // the same bits in every kernel (sw_rows.hpp)
     speccomb = cola + strrat * colb;
     R specparm = fdiv(cola, speccomb);
     const R oneminus = (R)(1.0 - 1.e-6);
