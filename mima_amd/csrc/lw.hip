@@ -173,33 +173,17 @@ __global__ __launch_bounds__(256) void lw_prep_kernel(ColumnInputs in, LwWork w,
     }
 }
 
-// per-column part of the prep (one thread per column): laytrop and the
-// precipitable water from the column's water and dry-air totals, summed in
-// the reference's order (rrtmg_lw_rad.nomcica.f90:845-852)
+// per-column part of the prep (lw_column_sums): laytrop, precipitable water,
+// surface temperature
 __global__ __launch_bounds__(256) void lw_column_kernel(ColumnInputs in, LwWork w)
 {
-    const int col = blockIdx.x * blockDim.x + threadIdx.x;
-    const int ncol = in.ncol, nlay = in.nlay;
-    if (col >= ncol) return;
-    const double amd = 28.9660, amw = 18.0160, amdw = 1.607793, avogad = 6.02214199e+23, grav = 9.8066;
-    double amttl = 0.0, wvttl = 0.0;
-    int laytrop = 0;
-    for (int lay = 0; lay < nlay; ++lay) {
-        const size_t ix = (size_t)lay * ncol + col;
-        double pz0 = in.plev[ix], pz1 = in.plev[ix + ncol];
-        double h2o = in.h2o[ix];
-        double wkl1 = in.vmr ? h2o : (h2o / (1.0 - h2o)) * amdw;
-        double amm = (1.0 - wkl1) * amd + wkl1 * amw;
-        double coldry = (pz0 - pz1) * 1.e3 * avogad / (1.e2 * grav * amm * (1.0 + wkl1));
-        wkl1 = coldry * wkl1;
-        amttl = amttl + coldry + wkl1;
-        wvttl = wvttl + wkl1;
-        if (log(in.play[ix]) > 4.56) ++laytrop;
-    }
-    double wvsh = (amw * wvttl) / (amd * amttl);
-    double pwvcm = wvsh * (1.e3 * in.plev[col]) / (1.e2 * grav);
-    w.laytrop[col] = laytrop;
-    w.colscal[col] = pwvcm;
+    const int col = blockIdx.x * 64 + ((int)threadIdx.x & 63), ncol = in.ncol;
+    const LwColumn r = lw_column_sums(in.plev, in.h2o, in.vmr, w.ipk, ncol, in.nlay, min(col, ncol - 1));
+    if (threadIdx.x >= 64 || col >= ncol) return;
+    const double amd = 28.9660, amw = 18.0160, grav = 9.8066;
+    const double wvsh = (amw * r.wvttl) / (amd * r.amttl);
+    w.laytrop[col] = r.laytrop;
+    w.colscal[col] = wvsh * (1.e3 * in.plev[col]) / (1.e2 * grav);
     w.colscal[(size_t)ncol + col] = in.tsfc[col];
 }
 
@@ -668,7 +652,7 @@ template <typename Real>
 static hipError_t launch_lw_t(const ColumnInputs &in, const LwOutputs &out, const LwWork &w, const LwDevTables &t,
                               double heatfac, bool smooth, hipStream_t s, hipEvent_t *ev)
 {
-    const int nb = (in.ncol + 255) / 256;
+    const int nb = (in.ncol + 63) / 64;
     const int nbl = (int)(((size_t)in.nlay * in.ncol + 255) / 256);
     if (ev) (void)hipEventRecord(ev[0], s);
     hipLaunchKernelGGL(lw_prep_kernel<Real>, dim3(nbl), dim3(256), 0, s, in, w, t.cst);
@@ -701,7 +685,7 @@ static hipError_t launch_lw_t(const ColumnInputs &in, const LwOutputs &out, cons
 
 hipError_t launch_lw_prep(const ColumnInputs &in, const LwWork &w, const LwDevTables &t, int mode, hipStream_t s)
 {
-    const int nb = (in.ncol + 255) / 256;
+    const int nb = (in.ncol + 63) / 64;
     const int nbl = (int)(((size_t)in.nlay * in.ncol + 255) / 256);
     if (mode == 1)
         hipLaunchKernelGGL(lw_prep_kernel<float>, dim3(nbl), dim3(256), 0, s, in, w, t.cst);

@@ -59,6 +59,47 @@ __device__ __forceinline__ void lw_load_layer(LwLayer<Real> &c, const Real *__re
     c.indlay = unpack_indlay(w);
 }
 
+// Per-column part of the LW preps: laytrop, and the column's water and dry-air
+// totals (rrtmg_lw_rad.nomcica.f90:845-852).  A block of 256 threads takes 64
+// columns, its four waves a quarter of the layers each (one thread per column
+// ran 40 divisions and logarithms in a chain: 37 us at 8192 x 40); the quarters
+// are added in order.  Lower layers are those whose forfac index is not the
+// upper atmosphere's, 3.  Valid in the first wave.
+struct LwColumn {
+    int laytrop;
+    double amttl, wvttl;
+};
+__device__ __forceinline__ LwColumn lw_column_sums(const double *__restrict__ plev, const double *__restrict__ h2o,
+                                                   bool vmr, const int *__restrict__ ipk, int ncol, int nlay, int col)
+{
+    const double amd = 28.9660, amw = 18.0160, amdw = 1.607793, avogad = 6.02214199e+23, grav = 9.8066;
+    __shared__ LwColumn part[256];
+    const int q = (int)threadIdx.x >> 6;
+    LwColumn r{0, 0.0, 0.0};
+#pragma unroll 4
+    for (int lay = q * nlay / 4; lay < (q + 1) * nlay / 4; ++lay) {
+        const size_t ix = (size_t)lay * ncol + col;
+        const double pz0 = plev[ix], pz1 = plev[ix + ncol], h = h2o[ix];
+        double wkl1 = vmr ? h : (h / (1.0 - h)) * amdw;
+        const double amm = (1.0 - wkl1) * amd + wkl1 * amw;
+        const double coldry = (pz0 - pz1) * 1.e3 * avogad / (1.e2 * grav * amm * (1.0 + wkl1));
+        wkl1 = coldry * wkl1;
+        r.amttl = r.amttl + coldry + wkl1;
+        r.wvttl = r.wvttl + wkl1;
+        r.laytrop += unpack_indf(ipk[ix]) != 3;
+    }
+    part[threadIdx.x] = r;
+    __syncthreads();
+    if (q == 0)
+        for (int k = 1; k < 4; ++k) {
+            const LwColumn o = part[threadIdx.x + 64 * k];
+            r.laytrop += o.laytrop;
+            r.amttl = r.amttl + o.amttl;
+            r.wvttl = r.wvttl + o.wvttl;
+        }
+    return r;
+}
+
 template <typename Real>
 struct LTab {
     const Real *__restrict__ t;

@@ -199,34 +199,20 @@ __global__ __launch_bounds__(256) void lw_vjp_prep_kernel(ColumnInputs in, VjpCo
     }
 }
 
-// per-column part of the prep (one thread per column): laytrop, the column
-// water and dry-air totals (the forward's arithmetic and summation order),
-// precipitable water and surface temperature
+// per-column part of the prep (lw_column_sums): laytrop, the column water and
+// dry-air totals, precipitable water and surface temperature
 __global__ __launch_bounds__(256) void lw_vjp_column_kernel(ColumnInputs in, LwVjpWork w)
 {
-    const int col = blockIdx.x * blockDim.x + threadIdx.x;
-    const int ncol = in.ncol, nlay = in.nlay;
-    if (col >= ncol) return;
-    const double amd = 28.9660, amw = 18.0160, amdw = 1.607793, avogad = 6.02214199e+23, grav = 9.8066;
-    double amttl = 0.0, wvttl = 0.0;
-    int laytrop = 0;
-    for (int lay = 0; lay < nlay; ++lay) {
-        const size_t ix = (size_t)lay * ncol + col;
-        const double h = in.h2o[ix], pz0 = in.plev[ix], pz1 = in.plev[ix + ncol];
-        double wkl1 = (h / (1.0 - h)) * amdw;
-        const double amm = (1.0 - wkl1) * amd + wkl1 * amw;
-        const double coldry = ((pz0 - pz1) * 1.e3 * avogad) / (1.e2 * grav * amm * (1.0 + wkl1));
-        wkl1 = coldry * wkl1;
-        amttl = amttl + coldry + wkl1;
-        wvttl = wvttl + wkl1;
-        if (log(in.play[ix]) > 4.56) ++laytrop;
-    }
-    const double wvsh = (amw * wvttl) / (amd * amttl);
-    w.laytrop[col] = laytrop;
+    const int col = blockIdx.x * 64 + ((int)threadIdx.x & 63), ncol = in.ncol;
+    const LwColumn r = lw_column_sums(in.plev, in.h2o, false, w.ipk, ncol, in.nlay, min(col, ncol - 1));
+    if (threadIdx.x >= 64 || col >= ncol) return;
+    const double amd = 28.9660, amw = 18.0160, grav = 9.8066;
+    const double wvsh = (amw * r.wvttl) / (amd * r.amttl);
+    w.laytrop[col] = r.laytrop;
     w.colscal[col] = wvsh * (1.e3 * in.plev[col]) / (1.e2 * grav);
     w.colscal[(size_t)ncol + col] = in.tsfc[col];
-    w.colscal[(size_t)2 * ncol + col] = wvttl;
-    w.colscal[(size_t)3 * ncol + col] = amttl;
+    w.colscal[(size_t)2 * ncol + col] = r.wvttl;
+    w.colscal[(size_t)3 * ncol + col] = r.amttl;
 }
 
 
@@ -367,7 +353,7 @@ template <typename Real>
 static void launch_lw_vjp_prep_t(const ColumnInputs &in, const VjpCot &cot, const LwVjpWork &w,
                                  const LwDevTables &t, hipStream_t s)
 {
-    const int nb = (in.ncol + 255) / 256;
+    const int nb = (in.ncol + 63) / 64;
     const int nbl = (int)(((size_t)in.nlay * in.ncol + 255) / 256);
     hipLaunchKernelGGL(lw_vjp_prep_kernel<Real>, dim3(nbl), dim3(256), 0, s, in, cot, w, t.cst, t.heatfac);
     hipLaunchKernelGGL(lw_vjp_column_kernel, dim3(nb), dim3(256), 0, s, in, w);

@@ -138,25 +138,22 @@ __global__ __launch_bounds__(256) void sw_prep_kernel(ColumnInputs in, SwWork w,
     }
 }
 
-// per-column part of the prep (one thread per column, after the per-layer
-// part, whose packed indices hold jp): laytrop, the solar-source reference
-// layers and, where w.day is given, the list of day columns, which the band
-// kernel's lanes are filled from (a wave's columns in order; the order of the
-// waves does not matter, columns being independent)
+// per-column part of the prep (sw_column_refs): laytrop, the solar-source
+// reference layers and, where w.day is given, the list of day columns, which
+// the band kernel's lanes are filled from (64 columns in order; the order of
+// the blocks does not matter, columns being independent)
 __global__ __launch_bounds__(256) void sw_column_kernel(ColumnInputs in, SwWork w)
 {
-    const int col = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool day = col < in.ncol && in.coszen[col] >= 1.e-10;
-    if (w.day) {
+    const int col0 = blockIdx.x * 64, lane = (int)threadIdx.x & 63, col = col0 + lane;
+    if (w.day && threadIdx.x < 64) {
+        const bool day = col < in.ncol && in.coszen[col] >= 1.e-10;
         const unsigned long long m = __builtin_amdgcn_ballot_w64(day);
-        const int lane = (int)threadIdx.x & 63;
         int base = 0;
         if (lane == 0 && m) base = atomicAdd(w.items + 1, __popcll(m));
         base = __builtin_amdgcn_readfirstlane(base);
         if (day) w.day[base + __popcll(m & ((1ull << lane) - 1))] = col;
     }
-    if (col >= in.ncol) return;
-    sw_column_refs(in.play, w.ipk, in.ncol, in.nlay, col, w.laytrop + col, w.laysolfr);
+    sw_column_refs(w.ipk, in.ncol, in.nlay, col0, w.laytrop, w.laysolfr);
 }
 
 // contraction off, as in sw_rows.hpp
@@ -550,7 +547,7 @@ template <typename Real>
 static hipError_t launch_sw_t(const ColumnInputs &in, const SwOutputs &out, const SwWork &w, const SwDevTables &t,
                               bool smooth, hipStream_t s, hipEvent_t *ev)
 {
-    const int nb = (in.ncol + 255) / 256;
+    const int nb = (in.ncol + 63) / 64;
     const int nbl = (int)(((size_t)in.nlay * in.ncol + 255) / 256);
     if (ev) (void)hipEventRecord(ev[0], s);
     hipLaunchKernelGGL(reset_items_kernel, dim3(1), dim3(2), 0, s, w.items);
@@ -576,7 +573,7 @@ static hipError_t launch_sw_t(const ColumnInputs &in, const SwOutputs &out, cons
 
 hipError_t launch_sw_prep(const ColumnInputs &in, const SwWork &w, const SwDevTables &t, int mode, hipStream_t s)
 {
-    const int nb = (in.ncol + 255) / 256;
+    const int nb = (in.ncol + 63) / 64;
     const int nbl = (int)(((size_t)in.nlay * in.ncol + 255) / 256);
     if (mode == 1)
         hipLaunchKernelGGL((sw_prep_kernel<float, false>), dim3(nbl), dim3(256), 0, s, in, w, t.preflog, t.tref);

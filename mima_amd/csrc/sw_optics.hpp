@@ -73,44 +73,61 @@ __device__ __forceinline__ void sw_load_groups(SwLayer<Real> &c, const Real *__r
     c.indf = unpack_indf(w);
 }
 
-// Per-column part of the SW prep for column col (after the per-layer part,
-// whose packed indices ipk hold jp): laytrop and the solar-source reference
-// layer of each band, laysolfr[b * ncol + col].  Bands searching the lower
-// atmosphere (18-25) take min(lay+1, laytrop) at the last jp crossing of
-// layreffr, default laytrop; bands searching aloft (16, 17, 27, 28, 29) take
-// the last crossing above laytrop, default nlayers; band 26 uses laytrop
-// (e.g. rrtmg_sw_taumol.f90:292-295, 391-394, 494-496).  One pass over the
-// layers tests every band's crossing.
-__device__ __forceinline__ void sw_column_refs(const double *__restrict__ play, const int *__restrict__ ipk,
-                                               int ncol, int nlay, int col, int *__restrict__ laytrop_out,
-                                               int *__restrict__ laysolfr)
+// Per-column part of the SW preps (after the per-layer part, whose packed
+// indices ipk hold jp): laytrop and the solar-source reference layer of each
+// band, laysolfr[b * ncol + col].  Bands searching the lower atmosphere (18-25)
+// take min(lay+1, laytrop) at the last jp crossing of layreffr, default laytrop;
+// bands searching aloft (16, 17, 27, 28, 29) take the last crossing above
+// laytrop, default nlayers; band 26 uses laytrop (e.g. rrtmg_sw_taumol.f90:
+// 292-295, 391-394, 494-496).  A block of 256 threads takes 64 columns, its
+// waves a quarter of the layers each (one thread per column took 41 us at
+// 8192 x 40, most of it a logarithm per layer; the lower layers are those whose
+// forfac index is not the upper atmosphere's, 3).
+__device__ __forceinline__ void sw_column_refs(const int *__restrict__ ipk, int ncol, int nlay, int col0,
+                                               int *__restrict__ laytrop_out, int *__restrict__ laysolfr)
 {
-    int laytrop = 0;
-    for (int lay = 0; lay < nlay; ++lay)
-        if (log(play[(size_t)lay * ncol + col]) > 4.56) ++laytrop;
-    *laytrop_out = laytrop;
     constexpr int lowref[14] = {0, 0, 6, 3, 3, 8, 2, 6, 1, 2, 0, 0, 0, 0};
     constexpr int upref[14] = {18, 30, 0, 0, 0, 0, 0, 0, 0, 0, 0, 32, 58, 49};
-    int lsf[14];
+    __shared__ int part[4][15][64];
+    const int q = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63, col = min(col0 + lane, ncol - 1);
+    const int beg = q * nlay / 4, end = (q + 1) * nlay / 4;  // layers beg+1 .. end
+    int n = 0;
+#pragma unroll 4
+    for (int lay = beg; lay < end; ++lay) n += unpack_indf(ipk[(size_t)lay * ncol + col]) != 3;
+    part[q][14][lane] = n;
+    __syncthreads();
+    const int laytrop = part[0][14][lane] + part[1][14][lane] + part[2][14][lane] + part[3][14][lane];
+    int last[14];  // the last crossing in this quarter, 0: none
 #pragma unroll
-    for (int b = 0; b < 14; ++b) lsf[b] = upref[b] > 0 ? nlay : laytrop;
+    for (int b = 0; b < 14; ++b) last[b] = 0;
     const int uplo = max(laytrop + 1, 2);
-    int jp2 = 0, jp1 = unpack_jp(ipk[col]);  // jp of layers lay-2 and lay-1
-    for (int lay = 1; lay <= nlay; ++lay) {
-        const int jpc = lay < nlay ? unpack_jp(ipk[(size_t)lay * ncol + col]) : jp1;  // jp(lay), jp(nlay-1) on top
+    auto jp = [&](int lay) { return unpack_jp(ipk[(size_t)clampi(lay, 0, nlay - 1) * ncol + col]); };
+    int jp2 = jp(beg - 1), jp1 = jp(beg);  // jp of layers lay-1 and lay
+#pragma unroll 4
+    for (int lay = beg + 1; lay <= end; ++lay) {
+        const int jpc = jp(lay);  // jp of layer lay+1, jp(nlay) on top
 #pragma unroll
         for (int b = 0; b < 14; ++b) {
             if (upref[b] > 0) {
-                if (lay >= uplo && jp2 < upref[b] && jp1 >= upref[b]) lsf[b] = lay;
+                if (lay >= uplo && jp2 < upref[b] && jp1 >= upref[b]) last[b] = lay;
             } else if (lowref[b] > 0) {
-                if (lay <= laytrop && jp1 < lowref[b] && jpc >= lowref[b]) lsf[b] = min(lay + 1, laytrop);
+                if (lay <= laytrop && jp1 < lowref[b] && jpc >= lowref[b]) last[b] = lay;
             }
         }
         jp2 = jp1;
         jp1 = jpc;
     }
 #pragma unroll
-    for (int b = 0; b < 14; ++b) laysolfr[(size_t)b * ncol + col] = max(lsf[b], 1);
+    for (int b = 0; b < 14; ++b) part[q][b][lane] = last[b];
+    __syncthreads();
+    if (q > 0 || col0 + lane >= ncol) return;
+    laytrop_out[col] = laytrop;
+#pragma unroll
+    for (int b = 0; b < 14; ++b) {
+        const int l = max(max(part[0][b][lane], part[1][b][lane]), max(part[2][b][lane], part[3][b][lane]));
+        const int lsf = upref[b] > 0 ? (l ? l : nlay) : (l ? min(l + 1, laytrop) : laytrop);
+        laysolfr[(size_t)b * ncol + col] = max(lsf, 1);
+    }
 }
 
 // X(jb) for every SW band, for switches over compile-time band bodies

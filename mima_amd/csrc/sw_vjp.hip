@@ -150,14 +150,10 @@ __global__ __launch_bounds__(256) void sw_vjp_prep_kernel(ColumnInputs in, VjpCo
     }
 }
 
-// per-column part of the prep (one thread per column, after the per-layer
-// part, whose packed indices hold jp): laytrop and the solar-source reference
-// layers, as the forward prep
+// per-column part of the prep, as the forward's
 __global__ __launch_bounds__(256) void sw_vjp_column_kernel(ColumnInputs in, SwVjpWork w)
 {
-    const int col = blockIdx.x * blockDim.x + threadIdx.x;
-    if (col >= in.ncol) return;
-    sw_column_refs(in.play, w.ipk, in.ncol, in.nlay, col, w.laytrop + col, w.laysolfr);
+    sw_column_refs(w.ipk, in.ncol, in.nlay, (int)blockIdx.x * 64, w.laytrop, w.laysolfr);
 }
 
 template <typename Real>
@@ -209,7 +205,7 @@ template <typename Real>
 static void launch_sw_vjp_prep_t(const ColumnInputs &in, const VjpCot &cot, const SwVjpWork &w,
                                  const SwDevTables &t, hipStream_t s)
 {
-    const int nb = (in.ncol + 255) / 256;
+    const int nb = (in.ncol + 63) / 64;
     const int nbl = (int)(((size_t)in.nlay * in.ncol + 255) / 256);
     hipLaunchKernelGGL(sw_vjp_prep_kernel<Real>, dim3(nbl), dim3(256), 0, s, in, cot, w, t.preflog, t.tref,
                        t.heatfac);
