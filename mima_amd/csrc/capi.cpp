@@ -1752,7 +1752,6 @@ static int lw_vjp_impl(int ncol, int nlay, const double *play, const double *ple
     }
     const int mixed = g_prec == RRTMG_HIP_PREC_MIXED;
     const size_t rs = mixed ? sizeof(float) : sizeof(double);
-    if ((rc = check_lds(lw_vjp_lds_bytes(nlay, rs)))) return rc;
     size_t off = 0;
     const size_t o_dc = off; off = align_up(off + rs * LWF_STRIDE * n2);
     const size_t o_dd = off; off = align_up(off + rs * LW_DSTRIDE * n2);
@@ -1765,13 +1764,13 @@ static int lw_vjp_impl(int ncol, int nlay, const double *play, const double *ple
     const size_t o_gp = off; off = align_up(off + rs * 16 * 3 * n2);
     const size_t o_gl = off; off = align_up(off + rs * 16 * n3);
     const size_t o_gs = off; off = align_up(off + rs * 16 * 2 * ncol);
-    const int chunk = vjp_chunk((ncol + TILE_COLS - 1) / TILE_COLS * s->lw.tab.nwaves, lw_vjp_state_bytes(nlay, rs));
     const bool lds = mixed && s->lwd.lds;
-    const size_t ds_bytes = lds ? (size_t)lw_vjp_lds_grid(s->lwd.plan, ncol, s->lw.tab.nwaves) * LWV_WGW *
-                                      lw_vjp_lds_state_bytes(nlay)
-                                : (size_t)chunk * lw_vjp_state_bytes(nlay, rs);
-    const size_t o_ds = off; off = align_up(off + ds_bytes);
-    const size_t o_it = off; off = align_up(off + sizeof(int));
+    // a fused session's kernel has tables in LDS and rows of its own
+    const int kind = lw_vjp_kind(ncol, rs, s->lwd.plan.ncu, lds);
+    const int chunk = lw_vjp_grid(ncol, nlay, rs, s->lwd.plan.ncu, kind);
+    const size_t o_ds = off;
+    off = align_up(off + (size_t)chunk * (kind == LWV_LDS ? LWV_WGW : 1) * lw_vjp_row_bytes(nlay, rs, kind));
+    const size_t o_it = off; off = align_up(off + 8 * sizeof(int));
     const size_t o_bf = off; off = align_up(off + (fwd ? rs * 16 * 2 * n3 : 0));
     if ((rc = W.lw_vjp_work.ensure(off))) return fail(rc, "device workspace allocation failed");
     char *wb = (char *)W.lw_vjp_work.p;
@@ -1789,6 +1788,7 @@ static int lw_vjp_impl(int ncol, int nlay, const double *play, const double *ple
     w.gsc = wb + o_gs;
     w.dstate = wb + o_ds;
     w.chunk = chunk;
+    w.kind = kind;
     w.items = (int *)(wb + o_it);
     w.bflux = fwd ? wb + o_bf : nullptr;
     if (host) {
@@ -1822,7 +1822,7 @@ static int lw_vjp_impl(int ncol, int nlay, const double *play, const double *ple
     t.cst = s->lwd.cst;
     t.units = s->lwd.units;
     t.heatfac = s->lw.cst.heatfac;
-    t.bands_lds = s->lwd.bands_lds;
+    t.bands_fwd = s->lwd.bands_fwd;
     t.plan = s->lwd.plan;
     t.lds = lds;
     if (fused) {
@@ -1952,17 +1952,13 @@ int rrtmg_hip_fused_end(void *stream)
         FusedBand a;
         a.lin = L.in;
         a.lw = L.w;
-        a.lbands = L.t.bands_lds;
+        a.lbands = L.t.bands_fwd;
         a.plan = L.t.plan;
-        a.lnwaves = L.t.desc.nwaves;
-        const int ltiles = (L.in.ncol + TILE_COLS - 1) / TILE_COLS;
-        a.litems = (ltiles + FUSED_WGW - 1) / FUSED_WGW * a.lnwaves;
-        a.exp_off = L.t.desc.exp_tbl;
-        a.tfn_off = L.t.desc.tfn_tbl;
+        a.litems = (L.in.ncol + LW_TILE - 1) / LW_TILE * LW_TILE_ITEMS;
+        a.et_off = L.t.desc.et_tbl;
         a.plk_off = L.t.desc.totplnk;
         a.ltab = (const float *)L.t.tab;
         a.cst = L.t.cst;
-        a.lunits = L.t.units;
         a.sin = S.in;
         a.sw = S.w;
         a.sbands = S.t.bands;

@@ -21,35 +21,33 @@ namespace rrtmg {
 
 size_t fused_lds_bytes(const LwLdsPlan &plan, int sw_nlay)
 {
-    return std::max((size_t)plan.lds_bytes, (size_t)FUSED_WGW * sw_vjp_lds_bytes(sw_nlay, sizeof(float)));
+    return std::max((size_t)plan.fwd_lds_bytes, (size_t)FUSED_WGW * sw_vjp_lds_bytes(sw_nlay, sizeof(float)));
 }
 
 size_t fused_row_floats(int lw_nlay, int sw_nlay)
 {
-    return std::max(lw_vjp_lds_state_bytes(lw_nlay), sw_vjp_state_bytes(sw_nlay, sizeof(float))) / sizeof(float);
+    return std::max(lw_vjp_row_bytes(lw_nlay, sizeof(float), LWV_LDS), sw_vjp_state_bytes(sw_nlay, sizeof(float))) / sizeof(float);
 }
 
 int fused_grid(const LwLdsPlan &plan, int nitems) { return std::min(plan.ncu, nitems); }
 
-// each side's band body is a call of its own (lw_vjp_unit, sw_vjp_unit), so
-// that the register allocation of one body does not weigh on the other's;
-// lw_vjp_unit is also what the LW LDS-table backward kernel calls (bitwise
-// the same LW results), the SW backward band kernel inlines its body
+// the SW body is a call of its own, so that its registers do not weigh on the LW
+// body's; the LW arithmetic has the same bits wherever it is compiled
+// (lw_rows.hpp)
 
 // 8 waves per workgroup at up to 256 VGPRs: two waves per SIMD
 __global__ __launch_bounds__(64 * FUSED_WGW) __attribute__((amdgpu_waves_per_eu(2)))
 void fused_band_kernel(FusedBand a)
 {
-    extern __shared__ unsigned char smem_raw[];
+    extern __shared__ __align__(16) unsigned char smem_raw[];
     float *lds = (float *)smem_raw;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
     float *row = a.rows + ((size_t)blockIdx.x * FUSED_WGW + wave) * a.row_floats;
-    const int lnlay = a.lin.nlay;
-    const int ltiles = (a.lin.ncol + TILE_COLS - 1) / TILE_COLS;
+    float *ktab = (float *)(smem_raw + LW_ET_VECS * 16);
     const size_t sw_wave_lds = sw_vjp_lds_bytes(a.sin.nlay, sizeof(float)) / sizeof(float);
     __shared__ int s_item;
     const SwUnitArgs<float> sa = sw_unit_args<float>(a.sin, a.sw, a.sexp_off, a.stab);
-    const LwUnitArgs la = lw_unit_args(a.lin, a.lw, a.exp_off, a.tfn_off, a.plk_off, a.ltab, a.cst);
+    const LwUnitArgs la = lw_unit_args(a.lin, a.lw, a.plk_off, a.ltab, a.cst);
     int loaded = -1;  // the LW band whose k-tables LDS holds
     for (;;) {
         // (next_item synchronises the workgroup: every wave is done with the
@@ -57,32 +55,26 @@ void fused_band_kernel(FusedBand a)
         const int item = next_item(a.items, &s_item);
         if (item >= a.nitems) break;
         if (item < a.litems) {
-            const int group = item / a.lnwaves, r = item - group * a.lnwaves;
-            const int b = a.lunits[r].band;
+            const int tile = item / LW_TILE_ITEMS;
+            const LwTileSlot slot = LW_TILE_SLOTS.s[item - tile * LW_TILE_ITEMS];
+            const int b = slot.band - 1;
+            if (loaded < 0)  // a workgroup's first item: the LW items come before the SW ones
+                for (int i = threadIdx.x; i < LW_ET_VECS; i += 64 * FUSED_WGW)
+                    ((uint4 *)smem_raw)[i] = ((const uint4 *)(a.ltab + a.et_off))[i];
             if (b != loaded) {
-                const int t0 = a.plan.tab0[b], n = a.plan.tab0[b + 1] - t0;
-#pragma unroll 8
-                for (int i = threadIdx.x; i < n; i += 64 * FUSED_WGW) lds[i] = a.ltab[t0 + i];
+                lw_copy_tables(ktab, a.ltab, a.plan, b);
                 __syncthreads();
                 loaded = b;
             }
-            const int k = (r - a.plan.ubeg[b]) * FUSED_WGW + wave;
-            const int tile = group * FUSED_WGW + k / a.plan.upt[b];
-            if (tile >= ltiles) continue;
-            const WaveUnit u = a.lunits[a.plan.ubeg[b] + k % a.plan.upt[b]];
-            const LwBand B = a.lbands[b];
-            float *s3 = row, *s1 = row + (size_t)2 * lnlay * 64;
-#define LBODY(bb)                                                                                              \
-    case bb - 1:                                                                                               \
-        lw_vjp_unit<bb>(la, B, (lptr<const float>)lds, u, tile, lane, (gptr<float>)s1, (gptr<float>)s3);      \
-        break;
-            switch (b) {
-                LBODY(1) LBODY(2) LBODY(3) LBODY(4) LBODY(5) LBODY(6) LBODY(7) LBODY(8)
-                LBODY(9) LBODY(10) LBODY(11) LBODY(12) LBODY(13) LBODY(14) LBODY(15) LBODY(16)
+            const int cend = min((tile + 1) * LW_TILE, a.lin.ncol);
+            for (int k = wave; k < 16; k += FUSED_WGW) {
+                const int c0 = tile * LW_TILE + (slot.part * 16 + k) * slot.cpw;
+                if (c0 >= cend) break;
+                lw_vjp_unit_of(la, a.lbands, b, (lptr<const ExpTfn<float>>)smem_raw, (lptr<const float>)ktab, c0, cend,
+                               lane, (gptr<float>)row);
             }
-#undef LBODY
         } else {
-            loaded = -1;  // the SW units' LDS overlays the k-tables
+            loaded = -1;  // the SW units' LDS overlays the LW tables
             const int blk = (item - a.litems) * FUSED_WGW + wave;
             if (blk >= a.snunits) continue;
             const int tile = blk / a.snwaves;

@@ -91,16 +91,10 @@ inline int lw_lds_grid(const LwLdsPlan &p, int ncol, int nwaves)
     return nitems < p.ncu ? nitems : p.ncu;
 }
 inline size_t lw_lds_state_bytes(int nlay) { return sizeof(float) * 2 * (size_t)nlay * 64; }
-// the backward's LDS-table kernel: LWV_WGW waves per workgroup (at most 168
-// VGPRs, three waves per SIMD), per-wave rows of 3 x nlay x 64
-constexpr int LWV_WGW = 12;
-inline int lw_vjp_lds_grid(const LwLdsPlan &p, int ncol, int nwaves)
-{
-    const int ntiles = (ncol + TILE_COLS - 1) / TILE_COLS;
-    const int nitems = (ntiles + LWV_WGW - 1) / LWV_WGW * nwaves;
-    return nitems < p.ncu ? nitems : p.ncu;
-}
-__host__ __device__ inline size_t lw_vjp_lds_state_bytes(int nlay) { return sizeof(float) * 3 * (size_t)nlay * 64; }
+// waves of a workgroup of the backward's LDS-table kernel: two per SIMD, for
+// its 256 VGPRs (8192 x 40: 0.95 ms; twelve waves 1.35, sixteen 1.77, which
+// spill)
+constexpr int LWV_WGW = 8;
 
 struct LwDevTables {
     LwTables desc;
@@ -280,9 +274,12 @@ struct LwGrad {
 struct SwGrad {
     double *tlay, *h2o, *o3;
 };
+// the LW backward kernel: lw_vjp_band_lds_kernel, or lw_vjp_band_kernel with a
+// wave, or a workgroup of eight or four waves, per unit
+enum LwVjpKind { LWV_LDS, LWV_WAVE, LWV_GROUP8, LWV_GROUP4 };
 struct LwVjpWork {
-    void *dcoef = nullptr;    // [nlay][ncol][LWF_STRIDE] of Real: the field values
-    void *dder = nullptr;     // [nlay][ncol][LW_DSTRIDE] of Real: their nonzero derivatives (LW_DMASK)
+    void *dcoef = nullptr;    // [nlay][LWF_GROUPS][ncol][4] of Real: the field values
+    void *dder = nullptr;     // [nlay][LWD_GROUPS][ncol][4] of Real: their nonzero derivatives (LW_DMASK)
     void *tlev = nullptr;     // [nlay+1][ncol] of Real
     int *ipk = nullptr;       // [nlay][ncol]
     int *ilev = nullptr;      // [nlay+1][ncol]
@@ -292,12 +289,11 @@ struct LwVjpWork {
     void *gpart = nullptr;    // [16][3][nlay][ncol] of Real: per-band gradient (T, q, O3)
     void *glev = nullptr;     // [16][nlay+1][ncol] of Real: per-band gradient wrt level temperature
     void *gsc = nullptr;      // [16][2][ncol] of Real: per-band d/dtsfc and d/dpwvcm
-    void *dstate = nullptr;   // [rows][2][nlay][64] of Real: incoming downward radiance and upward source per wave
-                              // ([rows][3][nlay][64] with the transmittance for the LDS-table kernel)
-    int chunk = 0;            // wave units per backward band-kernel launch (rows of dstate)
+    void *dstate = nullptr;   // the waves' scratch rows, lw_vjp_row_bytes each
+    int chunk = 0;            // workgroups of the band kernel
     void *bflux = nullptr;    // [16][2][nlay+1][ncol] of Real: band fluxes of the recomputed forward, or NULL
-    int *items = nullptr;     // work-item counters of the persistent band kernels, 8
-    int kind = 0;             // which band kernel (lw_fwd_kind)
+    int *items = nullptr;     // work-item counters of the band kernel, 8
+    int kind = LWV_LDS;       // the band kernel
 };
 struct SwVjpWork {
     void *dcoef = nullptr;    // [nlay][ncol][SWF_STRIDE] of Real: the field values
@@ -406,9 +402,35 @@ __host__ __device__ inline size_t sw_vjp_state_bytes(int nlay, size_t real_size)
 {
     return real_size * (4 * (size_t)(nlay + 1) + 5 * (size_t)nlay) * 64;
 }
-inline size_t lw_vjp_state_bytes(int nlay, size_t real_size) { return real_size * 2 * (size_t)nlay * 64; }
-// LDS bytes of one backward band workgroup
-inline size_t lw_vjp_lds_bytes(int nlay, size_t real_size) { return real_size * ((size_t)nlay * 64 + 4 * 64); }
+// by the size of the call; a column's result is the same bits in each.  Small
+// calls leave the chip idle with a wave per unit (a layer is a long chain of
+// dependent loads), so the waves of a workgroup share its layers: eight of them
+// up to where one workgroup per unit fills the chip (FP32 128 x 40: 143 us,
+// four 167; FP64's registers allow four: 225), four up to FP32 2560 columns
+// (1024 x 40: 318 us; 3000 x 40: 679; the LDS-table kernel takes 652 up to
+// 4096 columns, four waves 878 there) and FP64 1536 (1024 x 40: 562 us against
+// 627 of a wave per unit, 4096 x 40: 1838 against 1402).
+inline int lw_vjp_kind(int ncol, size_t real_size, int ncu, bool lds)
+{
+    if (real_size == 8) return ncol < 1536 ? LWV_GROUP4 : LWV_WAVE;
+    if (lw_fwd_units(ncol) <= (size_t)ncu) return LWV_GROUP8;
+    return ncol < 2560 || !lds ? LWV_GROUP4 : LWV_LDS;
+}
+// a scratch row of a wave (three values of a lane's g-points, up to four, per
+// layer) or of a workgroup of several (six, and three sums, and one more value)
+__host__ __device__ inline size_t lw_vjp_row_bytes(int nlay, size_t real_size, int kind)
+{
+    return real_size * 64 * (kind <= LWV_WAVE ? 3 * 4 * (size_t)nlay : (6 * 4 + 3) * (size_t)nlay + 4);
+}
+// its workgroups: those that fit the chip at once, no more than there is work
+// for or than 2 GiB of rows hold
+inline int lw_vjp_grid(int ncol, int nlay, size_t real_size, int ncu, int kind)
+{
+    const size_t rows = VJP_SCRATCH_BYTES / (lw_vjp_row_bytes(nlay, real_size, kind) * (kind == LWV_LDS ? LWV_WGW : 1));
+    const size_t items = kind == LWV_LDS ? ((size_t)ncol + LW_TILE - 1) / LW_TILE * LW_TILE_ITEMS : lw_fwd_units(ncol);
+    const size_t fit = (size_t)ncu * (kind == LWV_WAVE ? 4 : kind == LWV_GROUP4 && real_size == 4 ? 2 : 1);
+    return (int)std::max<size_t>(1, std::min({rows, items, fit}));
+}
 __host__ __device__ inline size_t sw_vjp_lds_bytes(int nlay, size_t real_size) { return real_size * ((size_t)(nlay + 1) * 64 + 4 * 64); }
 
 // fwd: NULL, or the forward's outputs, formed from w.bflux (which the
@@ -438,20 +460,19 @@ hipError_t launch_sw_vjp_finish(const ColumnInputs &in, const SwGrad &out, const
 
 // The band phase of one LW and one SW backward (FP32, LW k-tables staged in
 // LDS) as one persistent kernel: workgroups of FUSED_WGW waves claim work
-// items from one counter, first the LW items (as the LW LDS-table kernel's,
-// FUSED_WGW tiles per group), then SW items of FUSED_WGW wave units each.
+// items from one counter, first the LW items (a band of a tile, as the LW
+// LDS-table kernel's), then SW items of FUSED_WGW wave units each.
 // Each wave has one global scratch row (row_floats floats) for either side.
 constexpr int FUSED_WGW = 8;
 struct FusedBand {
     ColumnInputs lin;
     LwVjpWork lw;
-    const LwBand *lbands;       // LDS-relative k-table offsets
+    const LwBand *lbands;       // LwDevTables::bands_fwd
     LwLdsPlan plan;
-    int lnwaves, litems;        // LW units per tile; LW items
-    int exp_off, tfn_off, plk_off;
+    int litems;                 // LW items
+    int et_off, plk_off;
     const float *ltab;
     const LwConst *cst;
-    const WaveUnit *lunits;
     ColumnInputs sin;
     SwVjpWork sw;
     const SwBand *sbands;

@@ -29,6 +29,7 @@
 #include "kernels.hpp"
 #include "lw_optics.hpp"
 #include "lw_rows.hpp"
+#include "lw_unit.hpp"
 #include "rrtmg_device.hpp"
 
 namespace rrtmg {
@@ -189,157 +190,6 @@ __global__ __launch_bounds__(256) void lw_column_kernel(ColumnInputs in, LwWork 
 
 // contraction off, as in lw_rows.hpp
 #pragma clang fp contract(off)
-
-// Sum of a column's g-points on its first lane: exact enough in FP64 (the sum
-// is rounded once to FP32, and FP64 differs from the reference's order by its
-// last digits only).
-template <int BAND, typename Real>
-__device__ __forceinline__ Real band_sum(const Real (&v)[LwLanes<BAND>::GC], int g0)
-{
-    using L = LwLanes<BAND>;
-    double s = 0.0;
-#pragma unroll
-    for (int j = 0; j < L::GC; ++j) {
-        const bool in = L::NG % L::GC == 0 || g0 + j < L::NG;
-        s = j == 0 ? (double)v[0] : in ? s + (double)v[j] : s;
-    }
-    if constexpr (L::LPC == 2) s = s + __shfl_down(s, 1);
-    if constexpr (L::LPC == 3) s = s + (__shfl_down(s, 1) + __shfl_down(s, 2));
-    if constexpr (L::LPC == 4) {
-        s = s + __shfl_down(s, 1);
-        s = s + __shfl_down(s, 2);
-    }
-    return (Real)s;
-}
-
-// (exp(-tau), tau transition function) entries of the 10000-interval tables
-template <typename Real>
-struct alignas(2 * sizeof(Real)) ExpTfn {
-    Real e, t;
-};
-
-// What a wave needs of one band and CPW columns from column c0 on, below cend.
-// ktab: the band's k-tables, at B's offsets (global, or a copy in LDS); ktab_b:
-// those of the upper atmosphere's major species (absb); tab: the packed global
-// buffer (Planck); et: the (exp, tfn) pairs (global or LDS), or NULL for the
-// smooth functions.
-template <int BAND, typename Real>
-struct LwUnit {
-    using L = LwLanes<BAND>;
-    static constexpr int NG = L::NG, GC = L::GC;
-    const ColumnInputs &in;
-    const LwWork &w;
-    const LwBand &B;
-    const Real *__restrict__ ktab, *__restrict__ ktab_b, *__restrict__ plk;
-    const ExpTfn<Real> *et;
-    const LwConst *__restrict__ cst;
-    int g0, col, laytrop;
-    bool first;  // the lane that stores the column's sums
-    Real secdiff;
-    __device__ __forceinline__ LwUnit(const ColumnInputs &in_, const LwWork &w_, const LwBand &B_,
-                                      const Real *ktab_, const Real *ktab_b_, const Real *tab,
-                                      const ExpTfn<Real> *et_, int plk_off, const LwConst *cst_, int c0, int cend,
-                                      int lane)
-        : in(in_), w(w_), B(B_), ktab(ktab_), ktab_b(ktab_b_), plk(tab + plk_off + (BAND - 1) * 181), et(et_), cst(cst_)
-    {
-        const int cl = lane / L::LPC;
-        g0 = (lane - cl * L::LPC) * GC;
-        const bool active = cl < L::CPW && c0 + cl < cend;
-        col = active ? c0 + cl : cend - 1;
-        first = active && g0 == 0;
-        laytrop = w.laytrop[col];
-        // diffusivity secant (rrtmg_lw_rtrnmr.f90:272-280)
-        double sd = 1.66;
-        if (!(BAND == 1 || BAND == 4 || BAND >= 10)) {
-            sd = B.a0 + B.a1 * exp(B.a2 * w.colscal[col]);
-            if (sd > 1.80) sd = 1.80;
-            if (sd < 1.50) sd = 1.50;
-        }
-        secdiff = (Real)sd;
-    }
-    __device__ __forceinline__ void load(LwLayer<Real> &c, int lev) const
-    {
-        lw_load_layer(c, (const Real *)w.coef, w.ipk, lev - 1, col, in.ncol, in.nlay);
-    }
-    __device__ __forceinline__ Real planklev(int lev) const
-    {
-        const int i = at32(w.ilev, (unsigned)(lev * in.ncol + col));
-        const Real f = at32((const Real *)w.tlev, (unsigned)(lev * in.ncol + col));
-        return fma(f, at32(plk, (unsigned)i) - at32(plk, (unsigned)(i - 1)), at32(plk, (unsigned)(i - 1)));
-    }
-    __device__ __forceinline__ Real planklay(const LwLayer<Real> &c) const
-    {
-        return fma(c.tlayfrac, at32(plk, (unsigned)c.indlay) - at32(plk, (unsigned)(c.indlay - 1)),
-                   at32(plk, (unsigned)(c.indlay - 1)));
-    }
-    // optical depths on the diffusivity path of layer lev, from its record
-    __device__ __forceinline__ void depths(const LwLayer<Real> &c, int lev, Real (&od)[GC]) const
-    {
-        const bool lower = lev <= laytrop;
-#pragma unroll
-        for (int j = 0; j < GC; ++j) od[j] = (Real)0;
-        lw_rows<BAND, Real, Real>(B, cst, c, lower, [&](auto where, int off, int r, Real wt) {
-            Real k[GC];
-            load_row<NG>(k, where == LW_ABSB ? ktab_b : ktab, (unsigned)(off + (r - 1) * NG + g0));
-#pragma unroll
-            for (int j = 0; j < GC; ++j) od[j] = fma(wt, k[j], od[j]);
-        });
-        const Real ta =
-            in.tauaer ? (Real)in.tauaer[((size_t)(BAND - 1) * in.nlay + (lev - 1)) * in.ncol + col] : (Real)0;
-#pragma unroll
-        for (int j = 0; j < GC; ++j) {
-            if constexpr (BAND == 4 || BAND == 7) od[j] = od[j] * lw_gfactor<BAND, Real>(g0 + j, lower);
-            od[j] = secdiff * (od[j] + ta);
-            if (od[j] < (Real)0) od[j] = (Real)0;
-        }
-    }
-    // Planck fractions of layer lev
-    __device__ __forceinline__ void fracs(const LwLayer<Real> &c, int lev, Real (&fr)[GC]) const
-    {
-#pragma unroll
-        for (int j = 0; j < GC; ++j) fr[j] = (Real)0;
-        lw_fracs<BAND, Real, Real>(B, cst, c, lev <= laytrop, [&](int off, int r, Real wt) {
-            Real k[GC];
-            load_row<NG>(k, ktab, (unsigned)(off + (r - 1) * NG + g0));
-#pragma unroll
-            for (int j = 0; j < GC; ++j) fr[j] = fma(wt, k[j], fr[j]);
-        });
-    }
-    // transmittance and transition function of an optical depth
-    __device__ __forceinline__ void transmit(Real od, Real &atr, Real &tf) const
-    {
-        if (!et) {  // smooth mode: the tabulated functions at every depth
-            const LwRT<Real> rt = lw_rt_exact(od, false);
-            atr = rt.atrans;
-            tf = rt.tf;
-        } else {
-            const ExpTfn<Real> x = et[tbl_index(od)];
-            const bool thin = od <= (Real)0.06;
-            atr = thin ? fma((Real)-0.5 * od, od, od) : (Real)1 - x.e;
-            tf = thin ? (Real)0.166667 * od : x.t;
-        }
-    }
-    // surface emission and reflection: downward radiances into upward ones
-    __device__ __forceinline__ void surface(const Real (&fr)[GC], Real (&rad)[GC]) const
-    {
-        const double tbound = w.colscal[(size_t)in.ncol + col];
-        const Real semiss = (Real)in.emis[(size_t)(BAND - 1) * in.ncol + col];
-        // surface Planck (rrtmg_lw_setcoef.f90:190-194), FP64
-        const int i = clampi((int)(tbound - 159.0), 1, 180);
-        const double f = tbound - 159.0 - (double)i;
-        const Real plankbnd =
-            (Real)((double)semiss * ((double)plk[i - 1] + f * ((double)plk[i] - (double)plk[i - 1])));
-#pragma unroll
-        for (int j = 0; j < GC; ++j) rad[j] = fma(fr[j], plankbnd, ((Real)1 - semiss) * rad[j]);
-    }
-    // band sum of the radiances at level lev (up: 1, down: 0)
-    __device__ __forceinline__ void store(const Real (&rad)[GC], int lev, int up) const
-    {
-        Real *bf = (Real *)w.bflux + (size_t)(2 * (BAND - 1) + 1 - up) * (in.nlay + 1) * in.ncol;
-        const Real s = band_sum<BAND>(rad, g0);
-        if (first) at32(bf, (unsigned)(lev * in.ncol + col)) = s;
-    }
-};
 
 // One unit by one wave (rrtmg_lw_rtrnmr.f90:483-716, clear sky): the downward
 // sweep keeps each layer's optical depths in the wave's scratch row,
@@ -538,14 +388,10 @@ __global__ __launch_bounds__(64 * WAVES)
 
 #pragma clang fp contract(fast)
 
-__constant__ constexpr LwTileSlots LW_TILE_SLOTS{};
-
 // FP32 kernel of the large calls: persistent 16-wave workgroups, one per CU,
 // with the (exp, tfn) pairs and one band's k-tables in LDS (absb of bands 3-5,
 // 75 KB, stays global).  Work item = one band of a tile of LW_TILE columns
-// (LwTileSlots), one unit of CPW columns per wave.  Each XCD claims the tiles
-// t = xcd (mod 8) from its own counter, so the bands that read a tile's
-// coefficients share an L2, and takes other XCDs' items when its own are gone.
+// (LwTileSlots), one unit of CPW columns per wave (lw_claim_tile_item).
 __global__ __launch_bounds__(1024) void lw_band_lds_kernel(ColumnInputs in, LwWork w,
                                                            const LwBand *__restrict__ bands_lds, LwLdsPlan plan,
                                                            size_t row_elems, int et_off, int plk_off,
@@ -553,10 +399,9 @@ __global__ __launch_bounds__(1024) void lw_band_lds_kernel(ColumnInputs in, LwWo
                                                            const LwConst *__restrict__ cst)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    constexpr int ET16 = (int)((2 * (NTBL + 1) * sizeof(float) + 15) / 16);
     ExpTfn<float> *et = (ExpTfn<float> *)smem_raw;
-    float *ktab = (float *)(smem_raw + ET16 * 16);
-    for (int i = threadIdx.x; i < ET16; i += 1024) ((uint4 *)smem_raw)[i] = ((const uint4 *)(tab + et_off))[i];
+    float *ktab = (float *)(smem_raw + LW_ET_VECS * 16);
+    for (int i = threadIdx.x; i < LW_ET_VECS; i += 1024) ((uint4 *)smem_raw)[i] = ((const uint4 *)(tab + et_off))[i];
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
     float *row = (float *)w.dstate + ((size_t)blockIdx.x * 16 + wave) * row_elems;
     const int ntiles = (in.ncol + LW_TILE - 1) / LW_TILE;
@@ -564,19 +409,7 @@ __global__ __launch_bounds__(1024) void lw_band_lds_kernel(ColumnInputs in, LwWo
     int loaded = -1, queue = 0;
     for (;;) {
         __syncthreads();
-        if (threadIdx.x == 0) {
-            int it = -1;
-            for (; queue < 8; ++queue) {
-                const int x = ((int)blockIdx.x + queue) & 7;
-                const int n = ((ntiles - x + 7) >> 3) * LW_TILE_ITEMS;
-                const int k = n > 0 ? atomicAdd(w.items + x, 1) : n;
-                if (k < n) {
-                    it = (x + 8 * (k / LW_TILE_ITEMS)) * LW_TILE_ITEMS + k % LW_TILE_ITEMS;
-                    break;
-                }
-            }
-            s_item = it;
-        }
+        if (threadIdx.x == 0) s_item = lw_claim_tile_item(w.items, ntiles, queue);
         __syncthreads();
         const int item = __builtin_amdgcn_readfirstlane(s_item);
         if (item < 0) return;
@@ -584,11 +417,7 @@ __global__ __launch_bounds__(1024) void lw_band_lds_kernel(ColumnInputs in, LwWo
         const LwTileSlot slot = LW_TILE_SLOTS.s[k];
         const int b = slot.band - 1;
         if (b != loaded) {
-            // the band's k-tables but for [cut0, cut1), absb where it stays global
-            const int t0 = plan.tab0[b], n = plan.tab0[b + 1] - t0, c0 = plan.cut0[b], c1 = plan.cut1[b];
-            for (int i = threadIdx.x; i < n / 4; i += 1024)
-                if (i < c0 / 4 || i >= c1 / 4)
-                    ((float4 *)ktab)[i < c0 / 4 ? i : i - (c1 - c0) / 4] = ((const float4 *)(tab + t0))[i];
+            lw_copy_tables(ktab, tab, plan, b);
             __syncthreads();
             loaded = b;
         }

@@ -119,14 +119,29 @@ struct Eta {
     int js;
 };
 
+__device__ __forceinline__ void set_val(float &x, float v) { x = v; }
+template <typename V>
+__device__ __forceinline__ void set_val(V &x, float v)
+{
+    x.v = v;
+}
 // binary-species parameter (e.g. rrtmg_lw_taumol.f90:496-509)
-template <typename V, typename S>
-__device__ __forceinline__ Eta<V> lw_eta(V cola, V colb, S rat, S mult)
+template <typename A, typename B, typename S>
+__device__ __forceinline__ auto lw_eta(const A &cola, const B &colb, S rat, S mult)
 {
 #pragma clang fp contract(off)  // the same bits in every kernel (lw_rows.hpp)
+    using V = decltype(cola + rat * colb);
     Eta<V> e;
     e.speccomb = cola + rat * colb;
     e.specparm = fdiv(cola, e.speccomb);
+    if constexpr (sizeof(S) == 4) {
+        // FP32: the value to its last bit (one rounding of the sum, the quotient
+        // corrected by its residual): the table row and, for a gradient, the
+        // slope depend on which side of a row's edge it falls
+        const S comb = fma(rat, val(colb), val(cola)), q = val(e.specparm);
+        set_val(e.speccomb, comb);
+        set_val(e.specparm, fma(fma(-q, comb, val(cola)), __builtin_amdgcn_rcpf(comb), q));
+    }
     const S oneminus = (S)(1.0 - 1.e-6);
     if (e.specparm >= oneminus) e.specparm = V(oneminus);
     V specmult = mult * e.specparm;
@@ -202,11 +217,11 @@ __device__ __forceinline__ V lw_pfrac(const LTab<Real> &T, int off, const Eta<V>
     return T(off, e.js) + e.fs * (T(off, e.js + 1) - T(off, e.js));
 }
 // column-amount adjustment of minor CO2/N2O (e.g. rrtmg_lw_taumol.f90:1314-1320)
-template <typename V, typename S>
-__device__ __forceinline__ V lw_adjcol(V col, V coldry, S chiref, S thresh, S base, S ex)
+template <typename V, typename W, typename S>
+__device__ __forceinline__ V lw_adjcol(const V &col, const W &coldry, S chiref, S thresh, S base, S ex)
 {
 #pragma clang fp contract(off)
-    V rat = fdiv((S)1.e20 * fdiv(col, coldry), chiref);
+    const V rat = fdiv((S)1.e20 * fdiv(col, coldry), chiref);
     if (rat > thresh) return (base + pow(rat - base, ex)) * chiref * coldry * (S)1.e-20;
     return col;
 }

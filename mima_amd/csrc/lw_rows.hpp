@@ -57,61 +57,88 @@ using LwOther = std::integral_constant<int, 0>;
 using LwAbsB = std::integral_constant<int, 1>;
 constexpr int LW_ABSB = 1;
 
-#define CHI(i, j) ((Real)at32(lw_cst<V>(cst->chi_mls, cst->chi_mls_f), (unsigned)(((j)-1) * 7 + ((i)-1))))
-#define RAT(NAME, e) ((Real)at32(lw_cst<V>(cst->NAME, cst->NAME##_f), (unsigned)(e)))
-#define CHIQ(a, b, j) ((Real)lw_cst<V>(cst->chi_ratio, cst->chi_ratio_f)[lw_chi_ratio_k<a, b, j>()])
+#define CHI(i, j) ((Real)at32(lw_cst<Real>(cst->chi_mls, cst->chi_mls_f), (unsigned)(((j)-1) * 7 + ((i)-1))))
+#define RAT(NAME, e) ((Real)at32(lw_cst<Real>(cst->NAME, cst->NAME##_f), (unsigned)(e)))
+#define CHIQ(a, b, j) ((Real)lw_cst<Real>(cst->chi_ratio, cst->chi_ratio_f)[lw_chi_ratio_k<a, b, j>()])
+
+// A backward caller, whose gradient would lose digits to the sum of weight
+// derivatives of opposite signs, takes the interpolations whole instead, by
+// further overloads of term and frac: a pair of rows (table, offset, row, step,
+// weight, fraction), three rows (table, offset, row, weight, three factors
+// that add up to one), the four rows of a minor species (table, offset, row,
+// rows per temperature, weight, temperature fraction, eta fraction, 0); frac
+// (offset, row, step, fraction).  Its type has a member type Whole.
+template <typename T, typename = void>
+struct LwTakesWhole : std::false_type {};
+template <typename T>
+struct LwTakesWhole<T, std::void_t<typename T::Whole>> : std::true_type {};
 
 // The rows of one (layer, column) of band BAND; the band formulas and their
 // reference lines are those of lw_gas.  Rows are 1-based as the reference's
 // indices.  The g-point factors of bands 4 and 7 aloft are lw_gfactor.
-template <int BAND, typename Real, typename V, typename FT>
-__device__ __forceinline__ void lw_rows(const LwBand &B, const LwConst *__restrict__ cst, const LwLayer<V> &c,
+template <int BAND, typename Real, typename L, typename FT>
+__device__ __forceinline__ void lw_rows(const LwBand &B, const LwConst *__restrict__ cst, const L &c,
                                         bool lower, FT &&term)
 {
     constexpr int NA = LW_NSPA[BAND - 1], NB = LW_NSPB[BAND - 1];
     const int ind0 = lower ? ((c.jp - 1) * 5 + (c.jt - 1)) * NA : ((c.jp - 13) * 5 + (c.jt - 1)) * NB;
     const int ind1 = lower ? (c.jp * 5 + (c.jt1 - 1)) * NA : ((c.jp - 12) * 5 + (c.jt1 - 1)) * NB;
     const int jp = c.jp;
-    auto pair = [&](auto k, int off, int row, int step, const V &m, const V &f) {  // m ((1-f) K[row] + f K[row+step])
-        const V mf = m * f;
-        term(k, off, row, m - mf);
-        term(k, off, row + step, mf);
+    auto pair = [&](auto k, int off, int row, int step, const auto &m, const auto &f) {  // m ((1-f) K[row] + f K[row+step])
+        if constexpr (LwTakesWhole<std::decay_t<FT>>::value) {
+            term(k, off, row, step, m, f);
+        } else {
+            const auto mf = m * f;
+            term(k, off, row, m - mf);
+            term(k, off, row + step, mf);
+        }
     };
-    auto four = [&](auto k, int off, const V &m) {
+    // m (k.w0 K[row] + k.w1 K[row+1] + k.w2 K[row+2])
+    auto three = [&](int off, int row, const auto &m, const auto &k) {
+        if constexpr (LwTakesWhole<std::decay_t<FT>>::value) {
+            term(LwOther{}, off, row, m, k.w0, k.w1, k.w2);
+        } else {
+            term(LwOther{}, off, row, m * k.w0);
+            term(LwOther{}, off, row + 1, m * k.w1);
+            term(LwOther{}, off, row + 2, m * k.w2);
+        }
+    };
+    auto four = [&](auto k, int off, const auto &m) {
         term(k, off, ind0 + 1, m * c.fac00);
         term(k, off, ind0 + 2, m * c.fac10);
         term(k, off, ind1 + 1, m * c.fac01);
         term(k, off, ind1 + 2, m * c.fac11);
     };
-    auto self = [&](const V &m) { pair(LwOther{}, B.selfref, c.inds, 1, m, c.selffrac); };
-    auto foreign = [&](const V &m) { pair(LwOther{}, B.forref, c.indf, 1, m, c.forfrac); };
-    auto minor1 = [&](int off, const V &m) { pair(LwOther{}, off, c.indm, 1, m, c.minorfrac); };
-    auto minor2 = [&](int off, int neta, const Eta<V> &e, const V &m) {
+    auto self = [&](const auto &m) { pair(LwOther{}, B.selfref, c.inds, 1, m, c.selffrac); };
+    auto foreign = [&](const auto &m) { pair(LwOther{}, B.forref, c.indf, 1, m, c.forfrac); };
+    auto minor1 = [&](int off, const auto &m) { pair(LwOther{}, off, c.indm, 1, m, c.minorfrac); };
+    auto minor2 = [&](int off, int neta, const auto &e, const auto &m) {
         const int r = e.js + neta * (c.indm - 1);
-        const V hi = m * c.minorfrac;
-        pair(LwOther{}, off, r, 1, m - hi, e.fs);
-        pair(LwOther{}, off, r + neta, 1, hi, e.fs);
+        if constexpr (LwTakesWhole<std::decay_t<FT>>::value) {
+            term(LwOther{}, off, r, neta, m, c.minorfrac, e.fs, 0);
+        } else {
+            const auto hi = m * c.minorfrac;
+            pair(LwOther{}, off, r, 1, m - hi, e.fs);
+            pair(LwOther{}, off, r + neta, 1, hi, e.fs);
+        }
     };
-    auto major3 = [&](int off, const Eta<V> &e, int ind, const V &fa, const V &fb) {
-        const LwEta3<Real, V> k = lw_eta3<Real>(e);
-        const V a = e.speccomb * fa, b = e.speccomb * fb;
+    auto major3 = [&](int off, const auto &e, int ind, const auto &fa, const auto &fb) {
+        const auto k = lw_eta3<Real>(e);
+        const auto a = e.speccomb * fa;
+        const auto b = e.speccomb * fb;
         const int r = ind + k.js;
-        term(LwOther{}, off, r, a * k.w0);
-        term(LwOther{}, off, r + 1, a * k.w1);
-        term(LwOther{}, off, r + 2, a * k.w2);
-        term(LwOther{}, off, r + 9, b * k.w0);
-        term(LwOther{}, off, r + 10, b * k.w1);
-        term(LwOther{}, off, r + 11, b * k.w2);
+        three(off, r, a, k);
+        three(off, r + 9, b, k);
     };
-    auto major_b = [&](int off, const Eta<V> &e, int ind, const V &fa, const V &fb) {
+    auto major_b = [&](int off, const auto &e, int ind, const auto &fa, const auto &fb) {
         pair(LwAbsB{}, off, ind + e.js, 1, e.speccomb * fa, e.fs);
         pair(LwAbsB{}, off, ind + e.js + 5, 1, e.speccomb * fb, e.fs);
     };
-    auto binary_lo = [&](const Eta<V> &e, const Eta<V> &e1) {
+    auto binary_lo = [&](const auto &e, const auto &e1) {
         major3(B.absa, e, ind0, c.fac00, c.fac10);
         major3(B.absa, e1, ind1, c.fac01, c.fac11);
     };
-    auto binary_hi = [&](const Eta<V> &e, const Eta<V> &e1) {
+    auto binary_hi = [&](const auto &e, const auto &e1) {
         major_b(B.absb, e, ind0, c.fac00, c.fac10);
         major_b(B.absb, e1, ind1, c.fac01, c.fac11);
     };
@@ -121,20 +148,20 @@ __device__ __forceinline__ void lw_rows(const LwBand &B, const LwConst *__restri
     };
     if constexpr (BAND == 1) {
         if (lower) {
-            const V cr = c.pavel < (Real)250 ? V((Real)1 - fdiv((Real)0.15 * ((Real)250 - c.pavel), (Real)154.4)) : V((Real)1);
+            const Real cr = c.pavel < (Real)250 ? (Real)1 - fdiv((Real)0.15 * ((Real)250 - c.pavel), (Real)154.4) : (Real)1;
             four(LwOther{}, B.absa, cr * c.colh2o);
             self(cr * c.selffac);
             foreign(cr * c.forfac);
             minor1(B.ka_mn2, cr * c.colbrd * c.scaleminorn2);
         } else {
-            const V cr = (Real)1 - (Real)0.15 * fdiv(c.pavel, (Real)95.6);
+            const Real cr = (Real)1 - (Real)0.15 * fdiv(c.pavel, (Real)95.6);
             four(LwAbsB{}, B.absb, cr * c.colh2o);
             foreign(cr * c.forfac);
             minor1(B.kb_mn2, cr * c.colbrd * c.scaleminorn2);
         }
     } else if constexpr (BAND == 2) {
         if (lower) {
-            const V cr = (Real)1 - fdiv((Real).05 * (c.pavel - (Real)100), (Real)900);
+            const Real cr = (Real)1 - fdiv((Real).05 * (c.pavel - (Real)100), (Real)900);
             four(LwOther{}, B.absa, cr * c.colh2o);
             self(cr * c.selffac);
             foreign(cr * c.forfac);
@@ -143,14 +170,14 @@ __device__ __forceinline__ void lw_rows(const LwBand &B, const LwConst *__restri
             foreign(c.forfac);
         }
     } else if constexpr (BAND == 3) {
-        const V adj = lw_adjcol(c.coln2o, c.coldry, CHI(4, jp + 1), (Real)1.5, (Real)0.5, (Real)0.65);
+        const auto adj = lw_adjcol(c.coln2o, c.coldry, CHI(4, jp + 1), (Real)1.5, (Real)0.5, (Real)0.65);
         if (lower) {
             binary_lo(lw_eta(c.colh2o, c.colco2, RAT(rat_h2oco2, jp), (Real)8),
                       lw_eta(c.colh2o, c.colco2, RAT(rat_h2oco2, jp + 1), (Real)8));
             cont();
             minor2(B.ka_mn2o, 9, lw_eta(c.colh2o, c.colco2, CHIQ(1, 2, 3), (Real)8), adj);
         } else {
-            const Eta<V> em = lw_eta(c.colh2o, c.colco2, CHIQ(1, 2, 13), (Real)4);
+            const auto em = lw_eta(c.colh2o, c.colco2, CHIQ(1, 2, 13), (Real)4);
             binary_hi(lw_eta(c.colh2o, c.colco2, RAT(rat_h2oco2, jp), (Real)4),
                       lw_eta(c.colh2o, c.colco2, RAT(rat_h2oco2, jp + 1), (Real)4));
             foreign(c.forfac);
@@ -184,7 +211,7 @@ __device__ __forceinline__ void lw_rows(const LwBand &B, const LwConst *__restri
         term(LwOther{}, B.cfc12, 1, c.wx3);
     } else if constexpr (BAND == 7) {
         if (lower) {
-            const Eta<V> em = lw_eta(c.colh2o, c.colo3, CHIQ(1, 3, 3), (Real)8);
+            const auto em = lw_eta(c.colh2o, c.colo3, CHIQ(1, 3, 3), (Real)8);
             binary_lo(lw_eta(c.colh2o, c.colo3, RAT(rat_h2oo3, jp), (Real)8),
                       lw_eta(c.colh2o, c.colo3, RAT(rat_h2oo3, jp + 1), (Real)8));
             cont();
@@ -194,7 +221,7 @@ __device__ __forceinline__ void lw_rows(const LwBand &B, const LwConst *__restri
             minor1(B.kb_mco2, lw_adjcol(c.colco2, c.coldry, CHI(2, jp + 1), (Real)3, (Real)2, (Real)0.79));
         }
     } else if constexpr (BAND == 8) {
-        const V adj = lw_adjcol(c.colco2, c.coldry, CHI(2, jp + 1), (Real)3, (Real)2, (Real)0.65);
+        const auto adj = lw_adjcol(c.colco2, c.coldry, CHI(2, jp + 1), (Real)3, (Real)2, (Real)0.65);
         if (lower) {
             four(LwOther{}, B.absa, c.colh2o);
             cont();
@@ -209,7 +236,7 @@ __device__ __forceinline__ void lw_rows(const LwBand &B, const LwConst *__restri
         term(LwOther{}, B.cfc12, 1, c.wx3);
         term(LwOther{}, B.cfc22adj, 1, c.wx4);
     } else if constexpr (BAND == 9) {
-        const V adj = lw_adjcol(c.coln2o, c.coldry, CHI(4, jp + 1), (Real)1.5, (Real)0.5, (Real)0.65);
+        const auto adj = lw_adjcol(c.coln2o, c.coldry, CHI(4, jp + 1), (Real)1.5, (Real)0.5, (Real)0.65);
         if (lower) {
             binary_lo(lw_eta(c.colh2o, c.colch4, RAT(rat_h2och4, jp), (Real)8),
                       lw_eta(c.colh2o, c.colch4, RAT(rat_h2och4, jp + 1), (Real)8));
@@ -255,7 +282,7 @@ __device__ __forceinline__ void lw_rows(const LwBand &B, const LwConst *__restri
         }
     } else if constexpr (BAND == 15) {
         if (lower) {
-            const Eta<V> em = lw_eta(c.coln2o, c.colco2, CHIQ(4, 2, 1), (Real)8);
+            const auto em = lw_eta(c.coln2o, c.colco2, CHIQ(4, 2, 1), (Real)8);
             binary_lo(lw_eta(c.coln2o, c.colco2, RAT(rat_n2oco2, jp), (Real)8),
                       lw_eta(c.coln2o, c.colco2, RAT(rat_n2oco2, jp + 1), (Real)8));
             cont();
@@ -275,15 +302,19 @@ __device__ __forceinline__ void lw_rows(const LwBand &B, const LwConst *__restri
 // The rows of the Planck fraction of one (layer, column) of band BAND: two of
 // the band's species parameter at a reference level, or one.  Bands 12 and 15
 // have none aloft (their optics are zero there).
-template <int BAND, typename Real, typename V, typename FF>
-__device__ __forceinline__ void lw_fracs(const LwBand &B, const LwConst *__restrict__ cst, const LwLayer<V> &c,
+template <int BAND, typename Real, typename L, typename FF>
+__device__ __forceinline__ void lw_fracs(const LwBand &B, const LwConst *__restrict__ cst, const L &c,
                                          bool lower, FF &&frac)
 {
-    auto pfrac = [&](int off, const Eta<V> &e) {
-        frac(off, e.js, (Real)1 - e.fs);
-        frac(off, e.js + 1, e.fs);
+    auto pfrac = [&](int off, const auto &e) {
+        if constexpr (LwTakesWhole<std::decay_t<FF>>::value) {
+            frac(off, e.js, 1, e.fs);
+        } else {
+            frac(off, e.js, (Real)1 - e.fs);
+            frac(off, e.js + 1, e.fs);
+        }
     };
-    auto flat = [&](int off) { frac(off, 1, V((Real)1)); };
+    auto flat = [&](int off) { frac(off, 1, (Real)1); };
     (void)cst;
     if constexpr (BAND == 3) {
         if (lower)

@@ -14,20 +14,17 @@
 //    radiance cotangents after folding the heating-rate cotangent into the
 //    fluxes; then a per-column kernel for laytrop, the column water and
 //    dry-air totals, precipitable water and surface temperature.
-//  * band (one wave per work unit, lane = (column, g) as in the forward):
-//    pass A, downward sweep (values), storing per layer the transmittance
-//    in LDS and the upward source and the incoming downward radiance in a
-//    per-wave global scratch row (so LDS does not cap occupancy); pass B,
-//    upward sweep, replacing the source by (source - incoming upward
-//    radiance); pass C, reverse of the upward sweep, top-down, leaving the
-//    adjoints of the upward source and of the transmittance (upward part) in
-//    place of those two; pass D, reverse of the surface term and of the downward sweep,
-//    bottom-up: the layer's optical depth and Planck fraction are recomputed
-//    as dual numbers (no g-point-by-level tape is kept), the local derivatives
-//    of transmittance and source with respect to optical depth, Planck
-//    fraction and Planck integrals are analytic (for table lookups, those of
-//    the functions the tables tabulate), and the per-lane gradient is reduced
-//    over the band's g-points.
+//  * band (lane = up to four g-points of a column, as in the forward): top-down,
+//    the downward radiances and the adjoints of the upward ones; bottom-up, the
+//    upward radiances, the adjoints of the downward ones and the layers' local
+//    terms.  The optical depths are kept between the sweeps; the gas optics'
+//    derivatives come from the weights of their table rows (lw_vjp_body.hpp),
+//    those of transmittance and source are analytic (for table lookups, those
+//    of the functions the tables tabulate).  What bounds it is VALU work: with a
+//    lane per g-point, four sweeps and every derivative carried by every
+//    coefficient it took 1746 us at 8192 x 40 in FP32 (32768 x 60: 10.1 ms),
+//    now 946 (5.05); FP64 4096 x 40 2.80 -> 1.40 ms.  The prep stores groups of
+//    four fields, a wave's side by side: 121 -> 38 us.
 //  * finish (one thread per (layer, column)): sums over bands in FP64 and
 //    the precipitable-water chain of the diffusivity angle.
 #include <hip/hip_runtime.h>
@@ -58,19 +55,23 @@ __global__ __launch_bounds__(256) void lw_vjp_prep_kernel(ColumnInputs in, VjpCo
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (size_t)nlay * ncol) return;
     const int lay = (int)(i / ncol), col = (int)(i - (size_t)lay * ncol);
-    Real *dco = (Real *)w.dcoef, *dde = (Real *)w.dder;
     Real *tlevf = (Real *)w.tlev;
     const double amd = 28.9660, amw = 18.0160, amdw = 1.607793, amdo = 0.603428;
     const double avogad = 6.02214199e+23, grav = 9.8066;
     const double stpfac = 296.0 / 1013.0;
-    // the value record and the derivative record of the (layer, column)
-    auto put = [&](int F, size_t ix, const D3 &x) {
-        dco[ix * LWF_STRIDE + F] = (Real)x.v;
-        Real *d = dde + ix * LW_DSTRIDE + der_offset(LW_DMASK, F);
-        const unsigned m = LW_DMASK[F];
-        int k = 0;
-        for (int j = 0; j < 3; ++j)
-            if (m & (1u << j)) d[k++] = (Real)x.d[j];
+    // the values and the derivatives of the (layer, column)
+    Real rec[LWF_STRIDE], der[LW_DSTRIDE];
+#pragma unroll
+    for (int f = LWF_COUNT; f < LWF_STRIDE; ++f) rec[f] = (Real)0;
+#pragma unroll
+    for (int f = der_offset(LW_DMASK, LWF_COUNT); f < LW_DSTRIDE; ++f) der[f] = (Real)0;
+    auto put = [&](auto field, const D3 &x) {
+        constexpr int F = decltype(field)::value, O = der_offset(LW_DMASK, F);
+        constexpr unsigned m = LW_DMASK[F];
+        rec[F] = (Real)x.v;
+        if constexpr ((m & 1u) != 0) der[O] = (Real)x.d[0];
+        if constexpr ((m & 2u) != 0) der[O + dmask_count(m & 1u)] = (Real)x.d[1];
+        if constexpr ((m & 4u) != 0) der[O + dmask_count(m & 3u)] = (Real)x.d[2];
     };
     if (lay == 0) {
         double tz0 = in.tlev[col];
@@ -154,33 +155,45 @@ __global__ __launch_bounds__(256) void lw_vjp_prep_kernel(ColumnInputs in, VjpCo
         if (colch4.v == 0.0) colch4 = 1.e-32 * coldry;
         const D3 colbrd = 1.e-20 * wbrodl;
         const double compfp = 1. - fp;
-        put(LWF_FAC10, ix, compfp * ft);
-        put(LWF_FAC00, ix, compfp * (1.0 - ft));
-        put(LWF_FAC11, ix, fp * ft1);
-        put(LWF_FAC01, ix, fp * (1.0 - ft1));
-        put(LWF_COLH2O, ix, colh2o);
-        put(LWF_COLCO2, ix, colco2);
-        put(LWF_COLO3, ix, colo3);
-        put(LWF_COLN2O, ix, coln2o);
-        put(LWF_COLCO, ix, colco);
-        put(LWF_COLCH4, ix, colch4);
-        put(LWF_COLO2, ix, colo2);
-        put(LWF_COLBRD, ix, colbrd);
-        put(LWF_SELFFAC, ix, colh2o * selffac);
-        put(LWF_SELFFRAC, ix, selffrac);
-        put(LWF_FORFAC, ix, colh2o * forfac);
-        put(LWF_FORFRAC, ix, forfrac);
-        put(LWF_MINORFRAC, ix, minorfrac);
-        put(LWF_SCALEMINOR, ix, scaleminor);
-        put(LWF_SCALEMINORN2, ix, scaleminorn2);
-        put(LWF_COLDRY, ix, coldry);
-        put(LWF_PAVEL, ix, D3(pavel));
-        put(LWF_WX1, ix, wx1);
-        put(LWF_WX2, ix, wx2);
-        put(LWF_WX3, ix, wx3);
-        put(LWF_WX4, ix, wx4);
-        put(LWF_TLAYFRAC, ix, tlayfrac);
+        put(std::integral_constant<int, LWF_FAC10>{}, compfp * ft);
+        put(std::integral_constant<int, LWF_FAC00>{}, compfp * (1.0 - ft));
+        put(std::integral_constant<int, LWF_FAC11>{}, fp * ft1);
+        put(std::integral_constant<int, LWF_FAC01>{}, fp * (1.0 - ft1));
+        put(std::integral_constant<int, LWF_COLH2O>{}, colh2o);
+        put(std::integral_constant<int, LWF_COLCO2>{}, colco2);
+        put(std::integral_constant<int, LWF_COLO3>{}, colo3);
+        put(std::integral_constant<int, LWF_COLN2O>{}, coln2o);
+        put(std::integral_constant<int, LWF_COLCO>{}, colco);
+        put(std::integral_constant<int, LWF_COLCH4>{}, colch4);
+        put(std::integral_constant<int, LWF_COLO2>{}, colo2);
+        put(std::integral_constant<int, LWF_COLBRD>{}, colbrd);
+        put(std::integral_constant<int, LWF_SELFFAC>{}, colh2o * selffac);
+        put(std::integral_constant<int, LWF_SELFFRAC>{}, selffrac);
+        put(std::integral_constant<int, LWF_FORFAC>{}, colh2o * forfac);
+        put(std::integral_constant<int, LWF_FORFRAC>{}, forfrac);
+        put(std::integral_constant<int, LWF_MINORFRAC>{}, minorfrac);
+        put(std::integral_constant<int, LWF_SCALEMINOR>{}, scaleminor);
+        put(std::integral_constant<int, LWF_SCALEMINORN2>{}, scaleminorn2);
+        put(std::integral_constant<int, LWF_COLDRY>{}, coldry);
+        put(std::integral_constant<int, LWF_PAVEL>{}, D3(pavel));
+        put(std::integral_constant<int, LWF_WX1>{}, wx1);
+        put(std::integral_constant<int, LWF_WX2>{}, wx2);
+        put(std::integral_constant<int, LWF_WX3>{}, wx3);
+        put(std::integral_constant<int, LWF_WX4>{}, wx4);
+        put(std::integral_constant<int, LWF_TLAYFRAC>{}, tlayfrac);
         w.ipk[ix] = pack_lw(jp, jt, jt1, indself, indfor, indminor, indlay);
+        // [lay][group][col][4]: a wave's store of a group is contiguous
+        struct alignas(16) Group {
+            Real x[4];
+        };
+        Group *gv = (Group *)w.dcoef + (size_t)lay * LWF_GROUPS * ncol + col;
+        Group *gd = (Group *)w.dder + (size_t)lay * LWD_GROUPS * ncol + col;
+#pragma unroll
+        for (int k = 0; k < LWF_GROUPS; ++k)
+            gv[(size_t)k * ncol] = {rec[4 * k], rec[4 * k + 1], rec[4 * k + 2], rec[4 * k + 3]};
+#pragma unroll
+        for (int k = 0; k < LWD_GROUPS; ++k)
+            gd[(size_t)k * ncol] = {der[4 * k], der[4 * k + 1], der[4 * k + 2], der[4 * k + 3]};
     }
 
     // level radiance cotangents: fluxes' own cotangents plus the heating rate
@@ -216,86 +229,83 @@ __global__ __launch_bounds__(256) void lw_vjp_column_kernel(ColumnInputs in, LwV
 }
 
 
-template <typename Real>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(Real) == 4 ? 3 : 1)))
-void lw_vjp_band_kernel(ColumnInputs in, LwVjpWork w, const LwBand *__restrict__ bands,
-                                                         int nwaves, int blk0, int nblocks, int exp_off, int tfn_off,
-                                                         int plk_off, const Real *__restrict__ tab,
-                                                         const LwConst *__restrict__ cst,
-                                                         const WaveUnit *__restrict__ units)
+// Tables in global memory: persistent workgroups of WAVES waves; work items (CPW
+// columns of a band) from a counter, band by band, the bands with most work
+// first.  One wave: lw_vjp_band_body; more: lw_vjp_band_layers.
+template <typename Real, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(sizeof(Real) == 4 || WAVES > 4 ? 2 : 1)))
+void lw_vjp_band_kernel(ColumnInputs in, LwVjpWork w, const LwBand *__restrict__ bands, size_t row_elems, int et_off,
+                        int plk_off, const Real *__restrict__ tab, const LwConst *__restrict__ cst)
 {
-    extern __shared__ unsigned char smem_raw[];
-    Real *smem = (Real *)smem_raw;
-    const int blk = xcd_block();
-    if (blk >= nblocks) return;
-    const int tile = (blk0 + blk) / nwaves;
-    const WaveUnit u = units[(blk0 + blk) % nwaves];
-    const LwBand B = bands[u.band];
-    Real *s3 = (Real *)w.dstate + (size_t)blk * 2 * in.nlay * 64;
-    Real *s1 = smem, *red = smem + (size_t)in.nlay * 64;
-#define BODY(b)                                                                                          \
-    case b - 1:                                                                                          \
-        lw_vjp_band_body<b, Real>(in, w, B, tab, tab, exp_off, tfn_off, plk_off, cst, u, tile, (int)threadIdx.x, \
-                                  s1, s3, red);                                                          \
-        break;
-    switch (u.band) {
-        BODY(1) BODY(2) BODY(3) BODY(4) BODY(5) BODY(6) BODY(7) BODY(8)
-        BODY(9) BODY(10) BODY(11) BODY(12) BODY(13) BODY(14) BODY(15) BODY(16)
+    __shared__ int s_item;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
+    const ExpTfn<Real> *et = et_off >= 0 ? (const ExpTfn<Real> *)(tab + et_off) : nullptr;
+    Real *row = (Real *)w.dstate + (size_t)blockIdx.x * row_elems;
+    const LwWork f = lw_vjp_forward(w);
+    for (;;) {
+        int item = __builtin_amdgcn_readfirstlane(next_item(w.items, &s_item));
+#define BODY(b)                                                                                                  \
+    {                                                                                                            \
+        const int n = (in.ncol + lw_cpw(b) - 1) / lw_cpw(b);                                                     \
+        if (item < n) {                                                                                          \
+            const LwVjpUnit<b, Real> q(                                                                          \
+                LwUnit<b, Real>(in, f, bands[b - 1], tab, tab, tab, et, plk_off, cst, item * lw_cpw(b), in.ncol, lane), w); \
+            if constexpr (WAVES == 1) lw_vjp_band_body(q, lane, row);                                            \
+            else lw_vjp_band_layers<WAVES>(q, wave, lane, row);                                                  \
+            continue;                                                                                            \
+        }                                                                                                        \
+        item -= n;                                                                                               \
     }
+        BODY(5) BODY(3) BODY(4) BODY(7) BODY(9) BODY(13) BODY(12) BODY(8)
+        BODY(1) BODY(6) BODY(15) BODY(16) BODY(11) BODY(2) BODY(10) BODY(14)
 #undef BODY
+        return;
+    }
 }
 
-// FP32 backward band kernel with the band's k-tables in LDS, scheduled as the
-// forward's lw_band_lds_kernel (persistent workgroups of LWV_WGW waves that
-// claim work items from a global counter and copy a band's k-tables into LDS
-// before its first item).  All three per-layer states of a wave live in its
-// global scratch row, [3][nlay][64].
-template <typename Real>
+// FP32 kernel of the large calls, scheduled as the forward's lw_band_lds_kernel
+// (persistent workgroups with the (exp, tfn) pairs and one band's k-tables in
+// LDS; work items from the XCDs' counters) with LWV_WGW waves, each of which
+// takes every LWV_WGW-th of an item's 16 units.
 __global__ __launch_bounds__(64 * LWV_WGW) void lw_vjp_band_lds_kernel(ColumnInputs in, LwVjpWork w,
                                                                        const LwBand *__restrict__ bands,
-                                                                       LwLdsPlan plan, int nwaves, int nitems,
-                                                                       int exp_off, int tfn_off, int plk_off,
-                                                                       const Real *__restrict__ tab,
-                                                                       const LwConst *__restrict__ cst,
-                                                                       const WaveUnit *__restrict__ units)
+                                                                       LwLdsPlan plan, int et_off, int plk_off,
+                                                                       const float *__restrict__ tab,
+                                                                       const LwConst *__restrict__ cst)
 {
-    static_assert(sizeof(Real) == 4, "FP32 only: the FP64 g-sum synchronises the workgroup");
-    extern __shared__ unsigned char smem_raw[];
-    Real *ktab = (Real *)smem_raw;
-    const int nlay = in.nlay;
-    const int ntiles = (in.ncol + TILE_COLS - 1) / TILE_COLS;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    ExpTfn<float> *et = (ExpTfn<float> *)smem_raw;
+    float *ktab = (float *)(smem_raw + LW_ET_VECS * 16);
+    for (int i = threadIdx.x; i < LW_ET_VECS; i += 64 * LWV_WGW)
+        ((uint4 *)smem_raw)[i] = ((const uint4 *)(tab + et_off))[i];
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = (int)threadIdx.x & 63;
-    Real *s3 = (Real *)w.dstate + ((size_t)blockIdx.x * LWV_WGW + wave) * 3 * nlay * 64;
-    Real *s1 = s3 + (size_t)2 * nlay * 64;
+    float *row = (float *)w.dstate +
+                 ((size_t)blockIdx.x * LWV_WGW + wave) * lw_vjp_row_bytes(in.nlay, 1, LWV_LDS);
+    const int ntiles = (in.ncol + LW_TILE - 1) / LW_TILE;
+    const LwUnitArgs ua = lw_unit_args(in, w, plk_off, tab, cst);
     __shared__ int s_item;
-    const LwUnitArgs ua = lw_unit_args(in, w, exp_off, tfn_off, plk_off, tab, cst);
-    int loaded = -1;
+    int loaded = -1, queue = 0;
     for (;;) {
-        const int item = next_item(w.items, &s_item);
-        if (item >= nitems) break;
-        const int group = item / nwaves, r = item - group * nwaves;
-        const int b = units[r].band;
+        __syncthreads();
+        if (threadIdx.x == 0) s_item = lw_claim_tile_item(w.items, ntiles, queue);
+        __syncthreads();
+        const int item = __builtin_amdgcn_readfirstlane(s_item);
+        if (item < 0) return;
+        const int tile = item / LW_TILE_ITEMS;
+        const LwTileSlot slot = LW_TILE_SLOTS.s[item - tile * LW_TILE_ITEMS];
+        const int b = slot.band - 1;
         if (b != loaded) {
-            const int t0 = plan.tab0[b], n = plan.tab0[b + 1] - t0;
-#pragma unroll 8
-            for (int i = threadIdx.x; i < n; i += 64 * LWV_WGW) ktab[i] = tab[t0 + i];
+            lw_copy_tables(ktab, tab, plan, b);
             __syncthreads();
             loaded = b;
         }
-        const int k = (r - plan.ubeg[b]) * LWV_WGW + wave;
-        const int tile = group * LWV_WGW + k / plan.upt[b];
-        if (tile >= ntiles) continue;
-        const WaveUnit u = units[plan.ubeg[b] + k % plan.upt[b]];
-        const LwBand B = bands[b];
-#define BODY(bb)                                                                                              \
-    case bb - 1:                                                                                              \
-        lw_vjp_unit<bb>(ua, B, (lptr<const float>)ktab, u, tile, lane, (gptr<float>)s1, (gptr<float>)s3);    \
-        break;
-        switch (b) {
-            BODY(1) BODY(2) BODY(3) BODY(4) BODY(5) BODY(6) BODY(7) BODY(8)
-            BODY(9) BODY(10) BODY(11) BODY(12) BODY(13) BODY(14) BODY(15) BODY(16)
+        const int cend = min((tile + 1) * LW_TILE, in.ncol);
+        for (int k = wave; k < 16; k += LWV_WGW) {
+            const int c0 = tile * LW_TILE + (slot.part * 16 + k) * slot.cpw;
+            if (c0 >= cend) break;
+            lw_vjp_unit_of(ua, bands, b, (lptr<const ExpTfn<float>>)et, (lptr<const float>)ktab, c0, cend, lane,
+                           (gptr<float>)row);
         }
-#undef BODY
     }
 }
 
@@ -363,27 +373,27 @@ template <typename Real>
 static void launch_lw_vjp_band_t(const ColumnInputs &in, const LwVjpWork &w, const LwDevTables &t, bool smooth,
                                  hipStream_t s)
 {
-    const int ntiles = (in.ncol + TILE_COLS - 1) / TILE_COLS;
-    const size_t shmem = lw_vjp_lds_bytes(in.nlay, sizeof(Real));
-    const int nblocks = ntiles * t.desc.nwaves;
+    hipLaunchKernelGGL(reset_items_kernel, dim3(1), dim3(8), 0, s, w.items);
     if constexpr (sizeof(Real) == 4) {
-        if (t.lds && !smooth) {
-            const int nitems = (ntiles + LWV_WGW - 1) / LWV_WGW * t.desc.nwaves;
-            hipLaunchKernelGGL(reset_items_kernel, dim3(1), dim3(1), 0, s, w.items);
-            hipLaunchKernelGGL(lw_vjp_band_lds_kernel<Real>, dim3(lw_vjp_lds_grid(t.plan, in.ncol, t.desc.nwaves)),
-                               dim3(64 * LWV_WGW), (size_t)t.plan.lds_bytes, s, in, w, t.bands_lds, t.plan,
-                               t.desc.nwaves, nitems, t.desc.exp_tbl, t.desc.tfn_tbl, t.desc.totplnk,
-                               (const Real *)t.tab, t.cst, t.units);
+        if (w.kind == LWV_LDS) {
+            hipLaunchKernelGGL(lw_vjp_band_lds_kernel, dim3(w.chunk), dim3(64 * LWV_WGW), (size_t)t.plan.fwd_lds_bytes,
+                               s, in, w, t.bands_fwd, t.plan, t.desc.et_tbl, t.desc.totplnk, (const float *)t.tab,
+                               t.cst);
             return;
         }
     }
-    // launches of at most w.chunk wave units, each reusing the scratch rows
-    for (int b0 = 0; b0 < nblocks; b0 += w.chunk) {
-        const int nb_c = std::min(w.chunk, nblocks - b0);
-        hipLaunchKernelGGL(lw_vjp_band_kernel<Real>, dim3(xcd_grid(nb_c)), dim3(64), shmem, s, in, w, t.bands,
-                           t.desc.nwaves, b0, nb_c, smooth ? -1 : t.desc.exp_tbl, smooth ? -1 : t.desc.tfn_tbl,
-                           t.desc.totplnk, (const Real *)t.tab, t.cst, t.units);
+    const size_t row = lw_vjp_row_bytes(in.nlay, 1, w.kind);
+    const int et_off = smooth ? -1 : t.desc.et_tbl;
+#define LAUNCH(WAVES)                                                                                             \
+    hipLaunchKernelGGL((lw_vjp_band_kernel<Real, WAVES>), dim3(w.chunk), dim3(64 * WAVES), 0, s, in, w, t.bands, row, \
+                       et_off, t.desc.totplnk, (const Real *)t.tab, t.cst)
+    if (w.kind == LWV_GROUP4) LAUNCH(4);
+    if constexpr (sizeof(Real) == 4) {
+        if (w.kind == LWV_GROUP8) LAUNCH(8);
+    } else {
+        if (w.kind == LWV_WAVE) LAUNCH(1);
     }
+#undef LAUNCH
 }
 
 template <typename Real>

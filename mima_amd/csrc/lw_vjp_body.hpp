@@ -1,321 +1,600 @@
-// Backward band body of the clear-sky LW path (passes A-D, lw_vjp.hip) and
-// its loaders, shared by the LW backward band kernels and the fused
-// LW+SW forward+backward kernel (fused.hip).
+// Backward band body of the clear-sky LW path (two sweeps, lw_vjp.hip) and its
+// loaders, shared by the LW backward band kernels and the fused LW+SW
+// forward+backward kernel (fused.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include "kernels.hpp"
 #include "lw_optics.hpp"
+#include "lw_rows.hpp"
+#include "lw_unit.hpp"
+#include "mdual.hpp"
 #include "rrtmg_device.hpp"
 
 namespace rrtmg {
 
-// value (V = Real) or value and three derivatives (V = Dual<Real, 3>) of one
-// field: v, the field in the cell's value record; d, its first derivative in
-// the cell's derivative record.  MASK (bit 0: d/dT, 1: d/dq, 2: d/dO3, the
-// field's LW_DMASK entry) names the derivatives the field can have; the
-// others are known zeros, not stored, so the dual arithmetic on them folds
-// away at compile time.
-enum : unsigned { DT = 1u, DQ = 2u, DO = 4u };
-template <typename V, typename Real, unsigned MASK>
-struct DLoad;
-template <typename Real, unsigned MASK>
-struct DLoad<Real, Real, MASK> {
-    __device__ static Real get(const Real *__restrict__ v, const Real *__restrict__) { return v[0]; }
+// a layer's coefficients with the derivatives each can have (LW_DMASK)
+template <typename Real>
+struct LwLayerD {
+#define LWD(f, F) typename MField<Real, LW_DMASK[F]>::type f
+#define LWD_FIELDS(X)                                                                                              \
+    X(fac00, LWF_FAC00); X(fac01, LWF_FAC01); X(fac10, LWF_FAC10); X(fac11, LWF_FAC11);                            \
+    X(colh2o, LWF_COLH2O); X(colco2, LWF_COLCO2); X(colo3, LWF_COLO3); X(coln2o, LWF_COLN2O);                      \
+    X(colco, LWF_COLCO); X(colch4, LWF_COLCH4); X(colo2, LWF_COLO2); X(colbrd, LWF_COLBRD);                        \
+    X(selffac, LWF_SELFFAC); X(selffrac, LWF_SELFFRAC); X(forfac, LWF_FORFAC); X(forfrac, LWF_FORFRAC);            \
+    X(minorfrac, LWF_MINORFRAC); X(scaleminor, LWF_SCALEMINOR); X(scaleminorn2, LWF_SCALEMINORN2);                 \
+    X(coldry, LWF_COLDRY); X(pavel, LWF_PAVEL); X(wx1, LWF_WX1); X(wx2, LWF_WX2); X(wx3, LWF_WX3);                 \
+    X(wx4, LWF_WX4)
+    LWD_FIELDS(LWD);
+#undef LWD
+    Real tlayfrac;  // its derivative is 1
+    int jp, jt, jt1, inds, indf, indm, indlay;
 };
-template <typename Real, unsigned MASK>
-struct DLoad<Dual<Real, 3>, Real, MASK> {
-    __device__ static Dual<Real, 3> get(const Real *__restrict__ v, const Real *__restrict__ d)
-    {
-        Dual<Real, 3> r;
-        r.v = v[0];
-        r.d[0] = (MASK & DT) ? d[0] : (Real)0;
-        r.d[1] = (MASK & DQ) ? d[dmask_count(MASK & DT)] : (Real)0;
-        r.d[2] = (MASK & DO) ? d[dmask_count(MASK & (DT | DQ))] : (Real)0;
+
+// the field's derivatives, from der_offset on in the layer's groups of four
+template <unsigned M, typename Real, typename G>
+__device__ __forceinline__ auto lw_field_d(Real v, const G *g, int o)
+{
+    if constexpr (M == 0) {
+        return v;
+    } else {
+        MDual<Real, M> r;
+        r.v = v;
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            if (M >> k & 1u) {
+                r.d[k] = g[o / 4].x[o % 4];
+                ++o;
+            }
         return r;
     }
-};
+}
 
-// the layer's coefficients from the backward's records (values only when V
-// is Real: the derivative record is not read)
-template <typename V, typename Real>
-__device__ __forceinline__ void lw_load_layer_d(LwLayer<V> &c, const Real *__restrict__ dco,
-                                                const Real *__restrict__ dde, const int *__restrict__ ipk, int lay,
-                                                int col, int ncol)
-{
-    const unsigned ix = (unsigned)(lay * ncol + col);
-    const Real *vr = (const Real *)__builtin_assume_aligned(dco + (size_t)ix * LWF_STRIDE, 16);
-    const Real *dr = (const Real *)__builtin_assume_aligned(dde + (size_t)ix * LW_DSTRIDE, 16);
-#define LDD(f, F) c.f = DLoad<V, Real, LW_DMASK[F]>::get(vr + (F), dr + der_offset(LW_DMASK, F))
-    LDD(fac00, LWF_FAC00); LDD(fac01, LWF_FAC01); LDD(fac10, LWF_FAC10); LDD(fac11, LWF_FAC11);
-    LDD(colh2o, LWF_COLH2O); LDD(colco2, LWF_COLCO2); LDD(colo3, LWF_COLO3);
-    LDD(coln2o, LWF_COLN2O); LDD(colco, LWF_COLCO); LDD(colch4, LWF_COLCH4); LDD(colo2, LWF_COLO2);
-    LDD(colbrd, LWF_COLBRD); LDD(selffac, LWF_SELFFAC); LDD(selffrac, LWF_SELFFRAC);
-    LDD(forfac, LWF_FORFAC); LDD(forfrac, LWF_FORFRAC); LDD(minorfrac, LWF_MINORFRAC);
-    LDD(scaleminor, LWF_SCALEMINOR); LDD(scaleminorn2, LWF_SCALEMINORN2);
-    LDD(coldry, LWF_COLDRY); LDD(pavel, LWF_PAVEL); LDD(wx1, LWF_WX1); LDD(wx2, LWF_WX2);
-    LDD(wx3, LWF_WX3); LDD(wx4, LWF_WX4); LDD(tlayfrac, LWF_TLAYFRAC);
+// a layer's groups of four in the prep's two buffers, as loaded; groups a band
+// does not use are not loaded
+template <typename Real>
+struct LwGroupsD {
+    struct alignas(16) Group {
+        Real x[4];
+    };
+    Group v[LWF_GROUPS], d[LWD_GROUPS];
+    int ipk;
+    __device__ __forceinline__ void load(const Real *__restrict__ dco, const Real *__restrict__ dde,
+                                         const int *__restrict__ pk, int lay, int col, int ncol)
+    {
+        const Group *vb = (const Group *)dco + (size_t)lay * LWF_GROUPS * ncol;
+        const Group *db = (const Group *)dde + (size_t)lay * LWD_GROUPS * ncol;
+#pragma unroll
+        for (int k = 0; k < LWF_GROUPS; ++k)
+            v[k] = *(const Group *)((const char *)(vb + (size_t)k * ncol) + (LaneOffset<Real>)col * sizeof(Group));
+#pragma unroll
+        for (int k = 0; k < LWD_GROUPS; ++k)
+            d[k] = *(const Group *)((const char *)(db + (size_t)k * ncol) + (LaneOffset<Real>)col * sizeof(Group));
+        ipk = at32(pk, (unsigned)(lay * ncol + col));
+    }
+    __device__ __forceinline__ void unpack(LwLayerD<Real> &c) const
+    {
+#define LDD(f, F) c.f = lw_field_d<LW_DMASK[F], Real>(v[(F) / 4].x[(F) % 4], d, der_offset(LW_DMASK, F))
+        LWD_FIELDS(LDD);
 #undef LDD
-    const int w = at32(ipk, ix);
-    c.jp = unpack_jp(w);
-    c.jt = unpack_jt(w);
-    c.jt1 = unpack_jt1(w);
-    c.inds = unpack_inds(w);
-    c.indf = unpack_indf(w);
-    c.indm = unpack_indm(w);
-    c.indlay = unpack_indlay(w);
-}
-
-// transmittance and sources of one layer (rrtmg_lw_rtrnmr.f90:591-606) and,
-// for the backward, their derivatives with respect to the optical depth.
-// Values: the reference's thin-layer series below 0.06 and the tables above,
-// or (smooth mode, tables NULL) the tabulated functions themselves at every
-// depth; derivatives: always those of the smooth functions
-template <typename Real>
-struct LwLayerRT {
-    Real od, atrans, tf, datr, dtf;
+        c.tlayfrac = v[LWF_TLAYFRAC / 4].x[LWF_TLAYFRAC % 4];
+        c.jp = unpack_jp(ipk);
+        c.jt = unpack_jt(ipk);
+        c.jt1 = unpack_jt1(ipk);
+        c.inds = unpack_inds(ipk);
+        c.indf = unpack_indf(ipk);
+        c.indm = unpack_indm(ipk);
+        c.indlay = unpack_indlay(ipk);
+    }
 };
-template <typename Real>
-__device__ __forceinline__ LwLayerRT<Real> lw_layer_rt(Real secdiff, Real taug, const Real *__restrict__ exp_tbl,
-                                                       const Real *__restrict__ tfn_tbl, bool derivs)
+#undef LWD_FIELDS
+
+// contraction off, as in lw_rows.hpp
+#pragma clang fp contract(off)
+
+// sums over the lanes of a band, valid on the first one of each column
+template <int BAND, int N, typename Real>
+__device__ __forceinline__ void lw_lane_sums(Real (&v)[N])
 {
-    LwLayerRT<Real> r;
-    Real od = secdiff * taug;
-    if (od < (Real)0) od = (Real)0;
-    r.od = od;
-    if (!exp_tbl) {
-        const LwRT<Real> x = lw_rt_exact(od, derivs);
-        r.atrans = x.atrans;
-        r.tf = x.tf;
-        r.datr = x.datr;
-        r.dtf = x.dtf;
-    } else {
-        if (od <= (Real)0.06) {
-            r.atrans = od - (Real)0.5 * od * od;
-            r.tf = (Real)0.166667 * od;
-        } else {
-            const int itr = tbl_index(od);
-            r.atrans = (Real)1 - at32(exp_tbl, (unsigned)itr);
-            r.tf = at32(tfn_tbl, (unsigned)itr);
-        }
-        r.datr = r.dtf = (Real)0;
-        if (derivs) {
-            // the derivatives of the smooth functions that the series and the
-            // tables stand for, 1 - exp(-tau) and the tau transition
-            // function, at the same optical depth
-            const LwRT<Real> x = lw_rt_exact(od, true);
-            r.datr = x.datr;
-            r.dtf = x.dtf;
+    constexpr int LPC = LwLanes<BAND>::LPC;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        if constexpr (LPC == 2) v[i] = v[i] + __shfl_down(v[i], 1);
+        if constexpr (LPC == 3) v[i] = v[i] + (__shfl_down(v[i], 1) + __shfl_down(v[i], 2));
+        if constexpr (LPC == 4) {
+            v[i] = v[i] + __shfl_down(v[i], 1);
+            v[i] = v[i] + __shfl_down(v[i], 2);
         }
     }
-    return r;
 }
 
-// One band of one work unit of the backward (passes A-D, described at the top
-// of this file).  ktab: the k-tables (the packed global buffer, or the band's
-// copy in LDS with rebased offsets in B); tab: the packed global buffer
-// (transmittance and Planck tables).  s1: transmittance per layer, [nlay][64]
-// (LDS or global); s3: this wave's scratch row, incoming downward radiance
-// and upward source, [2][nlay][64]; red: [4][64] LDS entries for FP64 g-sums.
-template <int BAND, typename Real>
-__device__ __forceinline__ void lw_vjp_band_body(const ColumnInputs &in, const LwVjpWork &w, const LwBand &B,
-                                 const Real *__restrict__ ktab, const Real *__restrict__ tab, int exp_off,
-                                 int tfn_off, int plk_off, const LwConst *__restrict__ cst, WaveUnit u, int tile,
-                                 int lane, Real *__restrict__ s1, Real *__restrict__ s3, Real *red)
+// d/dtau of the transmittance 1 - exp(-tau) and of the tau transition function
+// (lw_rt_exact).  FP32: exp(-tau) from the hardware's exp2 with the product's
+// rounding error added back; the transition function's derivative, below 1.5,
+// from its series (sum (2n-1) 2 B_2n tau^(2n-2) / (2n)!, B the Bernoulli
+// numbers; the first term left out is 3e-9), above from
+// 2/tau^2 - 2 e/(1 - e)^2, which loses digits to cancellation below.
+template <typename Real>
+struct LwDRT {
+    Real datr, dtf;
+};
+__device__ __forceinline__ LwDRT<double> lw_drt(double od)
 {
-    constexpr int NG = lw_ng(BAND);
-    using V3 = Dual<Real, 3>;
-    const int ncol = in.ncol, nlay = in.nlay;
-    const int cl = lane / NG, g = lane - cl * NG;
-    const int col0 = tile * TILE_COLS + u.first_col + cl;
-    const bool active = cl < u.ncols && col0 < ncol;
-    const int col = active ? col0 : 0;
-    Real *__restrict__ s2 = s3 + (size_t)nlay * 64;
-    // s3: incoming downward radiance per layer, [nlay][64] in this wave's
-    // global scratch row (written in pass A, read back in pass D)
-    const Real *dco = (const Real *)w.dcoef, *dde = (const Real *)w.dder;
-    const Real *tlevf = (const Real *)w.tlev;
-    const Real *exp_tbl = exp_off >= 0 ? tab + exp_off : nullptr;
-    const Real *tfn_tbl = tfn_off >= 0 ? tab + tfn_off : nullptr;
-    const Real *plk = tab + plk_off + (BAND - 1) * 181;
-    LTab<Real> T{ktab, NG, g};
-    const size_t n2 = (size_t)nlay * ncol, n3 = (size_t)(nlay + 1) * ncol;
-    Real *gpart = (Real *)w.gpart + (size_t)(BAND - 1) * 3 * n2;
-    Real *glev = (Real *)w.glev + (size_t)(BAND - 1) * n3;
-    Real *gsc = (Real *)w.gsc + (size_t)(BAND - 1) * 2 * ncol;
+    const LwRT<double> x = lw_rt_exact(od, true);
+    return {x.datr, x.dtf};
+}
+__device__ __forceinline__ LwDRT<float> lw_drt(float od)
+{
+    const float log2e = 1.44269502f, log2e_lo = 1.92596303e-8f;
+    const float t = od * log2e, lo = fma(od, log2e, -t) + od * log2e_lo;
+    const float e0 = __builtin_amdgcn_exp2f(-t), e = fma(-0.693147181f * lo, e0, e0);
+    const float x2 = od * od;
+    float s = fma(3.4795e-10f, x2, -1.162518e-8f);
+    s = fma(s, x2, (float)(1. / 2661120.));
+    s = fma(s, x2, (float)(-1. / 86400.));
+    s = fma(s, x2, (float)(1. / 3024.));
+    s = fma(s, x2, (float)(-1. / 120.));
+    s = fma(s, x2, (float)(1. / 6.));
+    const float io = __builtin_amdgcn_rcpf(od), q = __builtin_amdgcn_rcpf(1.f - e);
+    return {e, od < 1.5f ? s : 2.f * fma(io, io, -(e * q) * q)};
+}
 
-    const int laytrop = w.laytrop[col];
-    const double pwvcm = w.colscal[col];
-    const double tbound = w.colscal[(size_t)ncol + col];
-    double sd = 1.66, dsd = 0.0;
-    if (!(BAND == 1 || BAND == 4 || BAND >= 10)) {
-        const double e = exp(B.a2 * pwvcm);
-        sd = B.a0 + B.a1 * e;
-        dsd = B.a1 * B.a2 * e;
-        if (sd > 1.80) { sd = 1.80; dsd = 0.0; }
-        if (sd < 1.50) { sd = 1.50; dsd = 0.0; }
+// Backward of one unit of a wave (its forward is that of u, and so are the band
+// fluxes, where w.bflux is given).
+//
+// Gradient with respect to a layer: the optical depth of g-point g is
+// sum_r W_r K_r[g] (lw_rows), so sum_g a_g dtau_g/dx = sum_r dW_r/dx (sum_g a_g
+// K_r[g]): the weights' derivatives are formed once for the lane's g-points
+// (Gather).
+template <int BAND, typename Real>
+struct LwVjpUnit {
+    using Unit = LwUnit<BAND, Real>;
+    static constexpr int GC = Unit::GC, NG = Unit::NG;
+    using Vec = GVec<GC, Real>;
+    const Unit u;
+    const LwVjpWork &w;
+    Real *gpart, *glev, *gsc;
+    const Real *cu, *cd;
+    size_t n2;
+    Real cband;
+    __device__ __forceinline__ LwVjpUnit(const Unit &u_, const LwVjpWork &w_) : u(u_), w(w_)
+    {
+        const size_t ncol = u.in.ncol, n3 = (size_t)(u.in.nlay + 1) * ncol;
+        n2 = (size_t)u.in.nlay * ncol;
+        gpart = (Real *)w.gpart + (size_t)(BAND - 1) * 3 * n2;
+        glev = (Real *)w.glev + (size_t)(BAND - 1) * n3;
+        gsc = (Real *)w.gsc + (size_t)(BAND - 1) * 2 * ncol;
+        cu = (const Real *)w.cot;
+        cd = cu + n3;
+        // radiance cotangents of this band: flux = fluxfac * sum_b 0.5 delwave_b sum_g rad
+        cband = (Real)(2.0 * asin(1.0) * 2.e4 * 0.5 * u.B.delwave);
     }
-    const Real secdiff = (Real)sd;
-    const Real semiss = (Real)in.emis[(size_t)(BAND - 1) * ncol + col];
-    const int indbound = clampi((int)(tbound - 159.0), 1, 180);
-    const double tbndfrac = tbound - 159.0 - (double)indbound;
-    const Real plankbnd = (Real)((double)semiss * ((double)plk[indbound - 1] +
-                                                   tbndfrac * ((double)plk[indbound] - (double)plk[indbound - 1])));
-    const Real dplankbnd = semiss * (plk[indbound] - plk[indbound - 1]);
-    auto planklev = [&](int lev) {
-        const int i = w.ilev[(size_t)lev * ncol + col];
-        const Real f = tlevf[(size_t)lev * ncol + col];
-        return plk[i - 1] + f * (plk[i] - plk[i - 1]);
+    __device__ __forceinline__ Real ru(int k) const { return at32(cu, (unsigned)(k * u.in.ncol + u.col)) * cband; }
+    __device__ __forceinline__ Real rd(int k) const { return at32(cd, (unsigned)(k * u.in.ncol + u.col)) * cband; }
+    // g-points past the band's end (dummies of its last lane) have no adjoints
+    __device__ __forceinline__ Real live(int j, Real x) const { return NG % GC == 0 || u.g0 + j < NG ? x : (Real)0; }
+    __device__ __forceinline__ Real plkslope(int i) const { return at32(u.plk, (unsigned)i) - at32(u.plk, (unsigned)(i - 1)); }
+    // What the rows of a layer add to its gradients g: an interpolation's
+    // derivative takes the difference of its rows, not the difference of their
+    // sums, which are many times larger (lw_rows).  S: sum over the lane's
+    // g-points of the adjoint times the row; a: the adjoints.
+    struct Gather {
+        using Whole = void;
+        const Real *ktab, *ktab_b;
+        const int g0;
+        const Real (&a)[GC];
+        Real (&g)[3];
+        template <int K>
+        __device__ __forceinline__ void row(Real (&k)[GC], std::integral_constant<int, K>, int off, int r) const
+        {
+            load_row<NG>(k, K == LW_ABSB ? ktab_b : ktab, (unsigned)(off + (r - 1) * NG + g0));
+        }
+        __device__ __forceinline__ Real dot(const Real (&k)[GC]) const
+        {
+            Real t = (Real)0;
+#pragma unroll
+            for (int j = 0; j < GC; ++j) t = fma(a[j], k[j], t);
+            return t;
+        }
+        __device__ __forceinline__ Real dot(const Real (&k)[GC], const Real (&l)[GC]) const  // of k - l
+        {
+            Real t = (Real)0;
+#pragma unroll
+            for (int j = 0; j < GC; ++j) t = fma(a[j], k[j] - l[j], t);
+            return t;
+        }
+        template <int K, typename W>
+        __device__ __forceinline__ void operator()(std::integral_constant<int, K> where, int off, int r, const W &m) const
+        {
+            Real k[GC];
+            row(k, where, off, r);
+            md_gather(g, dot(k), m);
+        }
+        template <int K, typename W, typename F>
+        __device__ __forceinline__ void operator()(std::integral_constant<int, K> where, int off, int r, int step, const W &m, const F &f) const
+        {
+            Real k0[GC], k1[GC];
+            row(k0, where, off, r);
+            row(k1, where, off, r + step);
+            const Real s0 = dot(k0), s1 = dot(k1, k0);
+            md_gather(g, fma(val(f), s1, s0), m);
+            md_gather(g, val(m) * s1, f);
+        }
+        template <int K, typename W, typename F>
+        __device__ __forceinline__ void operator()(std::integral_constant<int, K> where, int off, int r, const W &m, const F &w0, const F &,
+                                                   const F &w2) const
+        {
+            Real k0[GC], k1[GC], k2[GC];
+            row(k0, where, off, r);
+            row(k1, where, off, r + 1);
+            row(k2, where, off, r + 2);
+            const Real s1 = dot(k1), s0 = dot(k0, k1), s2 = dot(k2, k1);
+            md_gather(g, fma(val(w0), s0, fma(val(w2), s2, s1)), m);
+            md_gather(g, val(m) * s0, w0);
+            md_gather(g, val(m) * s2, w2);
+        }
+        template <int K, typename W, typename M, typename F>
+        __device__ __forceinline__ void operator()(std::integral_constant<int, K> where, int off, int r, int neta, const W &m, const M &mf,
+                                                   const F &fs, int) const
+        {
+            Real k0[GC], k1[GC], l0[GC], l1[GC];
+            row(k0, where, off, r);
+            row(k1, where, off, r + 1);
+            row(l0, where, off, r + neta);
+            row(l1, where, off, r + neta + 1);
+            const Real s0 = dot(k0), s1 = dot(k1, k0), d0 = dot(l0, k0), t1 = dot(l1, l0);
+            const Real low = fma(val(fs), s1, s0), up = fma(val(fs), t1 - s1, d0);
+            md_gather(g, fma(val(mf), up, low), m);
+            md_gather(g, val(m) * up, mf);
+            md_gather(g, val(m) * fma(val(mf), t1 - s1, s1), fs);
+        }
+        // the Planck fraction's rows
+        __device__ __forceinline__ void operator()(int, int, Real) const {}
+        template <typename F>
+        __device__ __forceinline__ void operator()(int off, int r, int step, const F &f) const
+        {
+            Real k0[GC], k1[GC];
+            row(k0, LwOther{}, off, r);
+            row(k1, LwOther{}, off, r + step);
+            md_gather(g, dot(k1, k0), f);
+        }
     };
-    auto plkslope = [&](int lev) {
-        const int i = w.ilev[(size_t)lev * ncol + col];
-        return plk[i] - plk[i - 1];
+    // a layer's local part: what one layer adds to the gradients, and the
+    // sweeps past it
+    struct Local {
+        Real g[3];           // T, q, O3 of the layer, over the lane's g-points
+        Real dn, up, sec;    // levels below and above; sum a_od od
     };
-    const double *tauaer = in.tauaer;
-    auto tau_a = [&](int lev) {
-        return tauaer ? (Real)tauaer[((size_t)(BAND - 1) * nlay + (lev - 1)) * ncol + col] : (Real)0;
-    };
-    // radiance cotangents of this band: flux = fluxfac * sum_b 0.5 delwave_b sum_g rad
-    const Real cband = (Real)(2.0 * asin(1.0) * 2.e4 * 0.5 * B.delwave);
-    const Real *cu = (const Real *)w.cot, *cd = cu + n3;
-    auto ru = [&](int k) { return active ? cu[(size_t)k * ncol + col] * cband : (Real)0; };
-    auto rd = [&](int k) { return active ? cd[(size_t)k * ncol + col] * cband : (Real)0; };
+    // p: the layer; od: optical depths; r, ar: downward radiances entering the layer and
+    // adjoints of the upward ones leaving it; rad, a: upward radiances entering
+    // it and adjoints of the downward ones leaving it, then those past it; af:
+    // the surface's adjoints of the lowest layer's Planck fractions, 0 elsewhere
+    __device__ __forceinline__ void load(LwGroupsD<Real> &p, int lev) const
+    {
+        p.load((const Real *)w.dcoef, (const Real *)w.dder, w.ipk, lev - 1, u.col, u.in.ncol);
+    }
+    __device__ __forceinline__ Local local(int lev, const LwGroupsD<Real> &p, const Vec &od, const Vec &r, const Vec &ar, const Vec &af,
+                                           Real plev_dn, Real plev_up, Real (&rad)[GC], Real (&a)[GC]) const
+    {
+        LwLayerD<Real> c;
+        p.unpack(c);
+        const bool lower = lev <= u.laytrop;
+        Real fr[GC], a_tg[GC], a_pf[GC];
+#pragma unroll
+        for (int j = 0; j < GC; ++j) fr[j] = (Real)0;
+        lw_fracs<BAND, Real>(u.B, u.cst, c, lower, [&](int off, int rr, const auto &wt) {
+            Real k[GC];
+            load_row<NG>(k, u.ktab, (unsigned)(off + (rr - 1) * NG + u.g0));
+#pragma unroll
+            for (int j = 0; j < GC; ++j) fr[j] = fma(val(wt), k[j], fr[j]);
+        });
+        const Real slope = plkslope(c.indlay), blay = fma(c.tlayfrac, slope, at32(u.plk, (unsigned)(c.indlay - 1)));
+        const Real dpdn = plev_dn - blay, dpup = plev_up - blay;
+        const Real ct = lev < u.in.nlay ? rd(lev) : (Real)0;
+        Local o{};
+        Real a_blay = (Real)0;
+#pragma unroll
+        for (int j = 0; j < GC; ++j) {
+            Real atr, tf;
+            u.transmit(od.x[j], atr, tf);
+            // the derivatives of the smooth functions that the series and the
+            // tables stand for, 1 - exp(-tau) and the transition function
+            const LwDRT<Real> x = lw_drt(od.x[j]);
+            const Real sdn = fma(tf, dpdn, blay), sup = fma(tf, dpup, blay);
+            const Real bbd = fr[j] * sdn, bbu = fr[j] * sup;
+            const Real a_bbd = a[j] * atr, a_bbu = ar.x[j] * atr;
+            const Real a_atr = fma(a[j], bbd - r.x[j], ar.x[j] * (bbu - rad[j]));
+            rad[j] = fma(bbu - rad[j], atr, rad[j]);
+            a[j] = fma(-a[j], atr, a[j]) + live(j, ct);
+            a_pf[j] = fma(a_bbd, sdn, fma(a_bbu, sup, af.x[j]));
+            const Real a_tf = fr[j] * fma(a_bbd, dpdn, a_bbu * dpup);
+            a_blay = fma(fr[j] * ((Real)1 - tf), a_bbd + a_bbu, a_blay);
+            o.dn = fma(a_bbd * fr[j], tf, o.dn);
+            o.up = fma(a_bbu * fr[j], tf, o.up);
+            const Real a_od = od.x[j] > (Real)0 ? fma(a_atr, x.datr, a_tf * x.dtf) : (Real)0;
+            o.sec = fma(a_od, od.x[j], o.sec);
+            a_tg[j] = a_od * u.secdiff;
+            if constexpr (BAND == 4 || BAND == 7) a_tg[j] = a_tg[j] * lw_gfactor<BAND, Real>(u.g0 + j, lower);
+        }
+        o.g[0] = a_blay * slope;
+        lw_rows<BAND, Real>(u.B, u.cst, c, lower, Gather{u.ktab, u.ktab_b, u.g0, a_tg, o.g});
+        lw_fracs<BAND, Real>(u.B, u.cst, c, lower, Gather{u.ktab, u.ktab, u.g0, a_pf, o.g});
+        return o;
+    }
+    // surface: rad and a of the downward sweep into those of the upward one;
+    // a_tb, af: the adjoints of the surface temperature and the Planck fractions
+    __device__ __forceinline__ void surface(const Real (&fr)[GC], Real (&rad)[GC], Real (&a)[GC], Real &a_tb,
+                                            Vec &af) const
+    {
+        const double tbound = u.w.colscal[(size_t)u.in.ncol + u.col];
+        const Real semiss = (Real)u.in.emis[(size_t)(BAND - 1) * u.in.ncol + u.col];
+        const Real dplankbnd = semiss * plkslope(clampi((int)(tbound - 159.0), 1, 180)), c0 = rd(0);
+        const Real emit = u.plankbnd();
+        u.surface(fr, rad);
+        a_tb = (Real)0;
+#pragma unroll
+        for (int j = 0; j < GC; ++j) {
+            af.x[j] = a[j] * emit;
+            a_tb = fma(a[j] * fr[j], dplankbnd, a_tb);
+            a[j] = fma(a[j], (Real)1 - semiss, live(j, c0));
+        }
+    }
+    __device__ __forceinline__ void store_layer(const Local &o, int lev) const
+    {
+        Real v[3] = {o.g[0], o.g[1], o.g[2]};
+        lw_lane_sums<BAND>(v);
+        if (u.first) {
+            const unsigned ix = (unsigned)((lev - 1) * u.in.ncol + u.col);
+            at32(gpart, ix) = v[0];
+            at32(gpart + n2, ix) = v[1];
+            at32(gpart + 2 * n2, ix) = v[2];
+        }
+    }
+    // gradient of level k from the layers above and below it
+    __device__ __forceinline__ void store_level(Real x, int k) const
+    {
+        const unsigned ix = (unsigned)(k * u.in.ncol + u.col);
+        Real v[1] = {x * plkslope(at32(w.ilev, ix))};
+        lw_lane_sums<BAND>(v);
+        if (u.first) at32(glev, ix) = v[0];
+    }
+    __device__ __forceinline__ void store_column(Real a_tb, Real a_sec) const
+    {
+        Real v[2] = {a_tb, a_sec};
+        lw_lane_sums<BAND>(v);
+        if (u.first) {
+            // a_sec holds sum a_od od = secdiff sum a_od tau
+            gsc[u.col] = v[0];
+            gsc[u.in.ncol + u.col] = v[1] / u.secdiff * u.dsecdiff();
+        }
+    }
+};
 
-    // band fluxes of the recomputed forward, when asked for (as the forward
-    // band kernel writes them; uniform branch)
-    Real *bf_up = w.bflux ? (Real *)w.bflux + (size_t)(BAND - 1) * 2 * n3 : nullptr;
-    Real *bf_dn = bf_up ? bf_up + n3 : nullptr;
-    if (bf_dn && active && g == 0) bf_dn[(size_t)nlay * ncol + col] = (Real)0;
-
-    // pass A: downward sweep
-    Real radld = (Real)0, fracs1 = (Real)0;
-    Real plev_up = planklev(nlay);
+// One unit by one wave.  Both sweeps of the forward have an adjoint that runs
+// the other way, and neither adjoint needs the forward's radiances but for the
+// local terms, so two sweeps do: top-down, the downward radiance and the
+// adjoint of the upward one; bottom-up, the upward radiance and the adjoint of
+// the downward one, with all local terms.  row: the wave's scratch,
+// [nlay][3][64][GC]: optical depths, incoming downward radiances, adjoints of
+// the upward radiances.
+template <int BAND, typename Real>
+__device__ __forceinline__ void lw_vjp_band_body(const LwVjpUnit<BAND, Real> q, int lane, Real *__restrict__ row)
+{
+    constexpr int GC = LwVjpUnit<BAND, Real>::GC;
+    using Vec = GVec<GC, Real>;
+    const auto &u = q.u;
+    const bool flux = q.w.bflux;
+    const int nlay = u.in.nlay;
+    auto at = [&](int lev, int k) -> Vec & { return at32((Vec *)row, (unsigned)(((lev - 1) * 3 + k) * 64 + lane)); };
+    Real rad[GC], a[GC], a_tb;  // radiances, the other direction's adjoints
+    Vec af;
     {
         LwLayer<Real> c;
+        Real fr[GC];
+        const Real top = q.ru(nlay);
+#pragma unroll
+        for (int j = 0; j < GC; ++j) {
+            rad[j] = (Real)0;
+            a[j] = q.live(j, top);
+        }
+        if (flux) u.store(rad, nlay, 0);
         for (int lev = nlay; lev >= 1; --lev) {
-            lw_load_layer_d<Real, Real>(c, dco, dde, w.ipk, lev - 1, col, ncol);
-            Real taug, plfrac;
-            lw_gas<BAND, Real>(B, T, cst, c, lev <= laytrop, taug, plfrac);
-            taug = taug + tau_a(lev);
-            const Real plev_dn = planklev(lev - 1);
-            const Real blay = plk[c.indlay - 1] + c.tlayfrac * (plk[c.indlay] - plk[c.indlay - 1]);
-            const LwLayerRT<Real> rt = lw_layer_rt(secdiff, taug, exp_tbl, tfn_tbl, false);
-            const Real bbd = plfrac * (blay + rt.tf * (plev_dn - blay));
-            const Real bbu = plfrac * (blay + rt.tf * (plev_up - blay));
-            at32(s1, (unsigned)((lev - 1) * 64 + lane)) = rt.atrans;
-            at32(s2, (unsigned)((lev - 1) * 64 + lane)) = bbu;
-            at32(s3, (unsigned)((lev - 1) * 64 + lane)) = radld;
-            radld = radld + (bbd - radld) * rt.atrans;
-            if (bf_dn) {
-                const Real sd = seg_sum(active ? radld : (Real)0, lane, g, NG, red);
-                if (active && g == 0) bf_dn[(size_t)(lev - 1) * ncol + col] = sd;
+            u.load(c, lev);
+            Vec od, r, s;
+            u.depths(c, lev, od.x);
+            u.fracs(c, lev, fr);
+            const Real blay = u.planklay(c), dplankdn = u.planklev(lev - 1) - blay, ct = q.ru(lev - 1);
+#pragma unroll
+            for (int j = 0; j < GC; ++j) {
+                Real atr, tf;
+                u.transmit(od.x[j], atr, tf);
+                r.x[j] = rad[j];
+                s.x[j] = a[j];
+                const Real bbd = fr[j] * fma(tf, dplankdn, blay);
+                rad[j] = fma(bbd - rad[j], atr, rad[j]);
+                a[j] = fma(-a[j], atr, a[j]) + q.live(j, ct);
             }
-            plev_up = plev_dn;
-            if (lev == 1) fracs1 = plfrac;
+            at(lev, 0) = od;
+            at(lev, 1) = r;
+            at(lev, 2) = s;
+            if (flux) u.store(rad, lev - 1, 0);
         }
+        q.surface(fr, rad, a, a_tb, af);
     }
-    // surface and pass B: upward sweep; keep source minus incoming radiance
-    Real radlu = fracs1 * plankbnd + ((Real)1 - semiss) * radld;
-    if (bf_up) {
-        const Real su = seg_sum(active ? radlu : (Real)0, lane, g, NG, red);
-        if (active && g == 0) bf_up[col] = su;
-    }
-    // the per-layer states are read one level ahead
-    Real s1n = at32(s1, (unsigned)lane), s2n = at32(s2, (unsigned)lane);
+    if (flux) u.store(rad, 0, 1);
+    Real a_sec = (Real)0, up = (Real)0, plev = u.planklev(0);
     for (int lev = 1; lev <= nlay; ++lev) {
-        const Real atr = s1n;
-        const Real dsrc = s2n - radlu;
-        if (lev < nlay) {
-            s1n = at32(s1, (unsigned)(lev * 64 + lane));
-            s2n = at32(s2, (unsigned)(lev * 64 + lane));
-        }
-        at32(s2, (unsigned)((lev - 1) * 64 + lane)) = dsrc;
-        radlu = radlu + dsrc * atr;
-        if (bf_up) {
-            const Real su = seg_sum(active ? radlu : (Real)0, lane, g, NG, red);
-            if (active && g == 0) bf_up[(size_t)lev * ncol + col] = su;
-        }
+        // (loaded here, before the layer's work; a layer ahead, their registers
+        // spill: 8192 x 40 1.01 -> 1.10 ms)
+        const Vec od = at(lev, 0), r = at(lev, 1), s = at(lev, 2);
+        LwGroupsD<Real> p;
+        q.load(p, lev);
+        const Real plev_up = u.planklev(lev);
+        const auto o = q.local(lev, p, od, r, s, af, plev, plev_up, rad, a);
+        plev = plev_up;
+#pragma unroll
+        for (int j = 0; j < GC; ++j) af.x[j] = (Real)0;
+        if (flux) u.store(rad, lev, 1);
+        q.store_layer(o, lev);
+        q.store_level(up + o.dn, lev - 1);
+        up = o.up;
+        a_sec = a_sec + o.sec;
     }
-    // pass C: reverse of the upward sweep (top-down)
-    Real a_ru = ru(nlay);
-    s1n = at32(s1, (unsigned)((nlay - 1) * 64 + lane));
-    s2n = at32(s2, (unsigned)((nlay - 1) * 64 + lane));
-    for (int lev = nlay; lev >= 1; --lev) {
-        const unsigned k = (unsigned)((lev - 1) * 64 + lane);
-        const Real atr = s1n, dsrc = s2n;
-        if (lev > 1) {
-            s1n = at32(s1, (unsigned)((lev - 2) * 64 + lane));
-            s2n = at32(s2, (unsigned)((lev - 2) * 64 + lane));
+    q.store_level(up, nlay);
+    q.store_column(a_tb, a_sec);
+}
+
+// One unit by a workgroup of WAVES waves, for calls too small to fill the chip
+// with waves: the layers' optics and local terms are shared out among the waves
+// and one wave runs the two sweeps between them.  row: the workgroup's scratch,
+// [nlay][6][64][GC] (optical depth, transmittance, the two sources, which the
+// incoming radiances replace, and the two adjoints), [nlay][3][64] (levels below
+// and above, sum a_od od of each layer) and [64][GC] (the surface's adjoints of
+// the Planck fractions).
+template <int WAVES, int BAND, typename Real>
+__device__ __forceinline__ void lw_vjp_band_layers(const LwVjpUnit<BAND, Real> q, int wave, int lane,
+                                                   Real *__restrict__ row)
+{
+    constexpr int GC = LwVjpUnit<BAND, Real>::GC;
+    using Vec = GVec<GC, Real>;
+    const auto &u = q.u;
+    const int nlay = u.in.nlay;
+    auto at = [&](int lev, int k) -> Vec & { return at32((Vec *)row, (unsigned)(((lev - 1) * 6 + k) * 64 + lane)); };
+    Real *sums = row + (size_t)nlay * 6 * 64 * GC;
+    auto sum = [&](int lev, int k) -> Real & { return at32(sums, (unsigned)(((lev - 1) * 3 + k) * 64 + lane)); };
+    for (int lev = nlay - wave; lev >= 1; lev -= WAVES) {
+        LwLayer<Real> c;
+        u.load(c, lev);
+        Vec od, atr, bbd, bbu;
+        Real fr[GC];
+        u.depths(c, lev, od.x);
+        u.fracs(c, lev, fr);
+        const Real blay = u.planklay(c), dn = u.planklev(lev - 1) - blay, up = u.planklev(lev) - blay;
+#pragma unroll
+        for (int j = 0; j < GC; ++j) {
+            Real tf;
+            u.transmit(od.x[j], atr.x[j], tf);
+            bbd.x[j] = fr[j] * fma(tf, dn, blay);
+            bbu.x[j] = fr[j] * fma(tf, up, blay);
         }
-        at32(s1, k) = a_ru * atr;   // adjoint of the upward source of layer lev
-        at32(s2, k) = a_ru * dsrc;  // adjoint of its transmittance, upward part
-        a_ru = a_ru * ((Real)1 - atr) + ru(lev - 1);
+        at(lev, 0) = od;
+        at(lev, 1) = atr;
+        at(lev, 2) = bbd;
+        at(lev, 3) = bbu;
     }
-    // reverse of the surface term
-    const Real a_fracs1 = a_ru * plankbnd;
-    Real a_tb = a_ru * fracs1 * dplankbnd;
-    Real a_rd = a_ru * ((Real)1 - semiss) + rd(0);
-    Real a_sec = (Real)0, pend_up = (Real)0;
-    // pass D: reverse of the downward sweep (bottom-up) with the layer's
-    // optical depth and Planck fraction recomputed as dual numbers
-    for (int lev = 1; lev <= nlay; ++lev) {
-        LwLayer<V3> c;
-        lw_load_layer_d<V3, Real>(c, dco, dde, w.ipk, lev - 1, col, ncol);
-        V3 tg3, pf3;
-        lw_gas<BAND, Real, V3>(B, T, cst, c, lev <= laytrop, tg3, pf3);
-        const Real tg = tg3.v + tau_a(lev), pf = pf3.v;
-        const Real plev_dn = planklev(lev - 1), plev_upv = planklev(lev);
-        const Real slope = plk[c.indlay] - plk[c.indlay - 1];
-        const Real blay = plk[c.indlay - 1] + c.tlayfrac.v * slope;
-        const LwLayerRT<Real> rt = lw_layer_rt(secdiff, tg, exp_tbl, tfn_tbl, true);
-        const Real dpdn = plev_dn - blay, dpup = plev_upv - blay;
-        const Real bbd = pf * (blay + rt.tf * dpdn);
-        const size_t k = (size_t)(lev - 1) * 64 + lane;
-        const Real a_bbd = a_rd * rt.atrans;
-        const Real a_atr = a_rd * (bbd - at32(s3, (unsigned)k)) + at32(s2, (unsigned)k);
-        const Real a_bbu = at32(s1, (unsigned)k);
-        a_rd = a_rd * ((Real)1 - rt.atrans) + (lev < nlay ? rd(lev) : (Real)0);
-        Real a_pf = a_bbd * (blay + rt.tf * dpdn) + a_bbu * (blay + rt.tf * dpup);
-        if (lev == 1) a_pf += a_fracs1;
-        const Real a_tf = pf * (a_bbd * dpdn + a_bbu * dpup);
-        const Real a_blay = pf * ((Real)1 - rt.tf) * (a_bbd + a_bbu);
-        const Real a_pdn = a_bbd * pf * rt.tf, a_pup = a_bbu * pf * rt.tf;
-        const Real a_od = rt.od > (Real)0 ? a_atr * rt.datr + a_tf * rt.dtf : (Real)0;
-        const Real a_tg = a_od * secdiff;
-        a_sec += a_od * tg;
-        Real v[4];
-        v[0] = a_tg * tg3.d[0] + a_pf * pf3.d[0] + a_blay * slope;
-        v[1] = a_tg * tg3.d[1] + a_pf * pf3.d[1];
-        v[2] = a_tg * tg3.d[2] + a_pf * pf3.d[2];
-        v[3] = (pend_up + a_pdn) * plkslope(lev - 1);  // level lev-1 is complete
-        pend_up = a_pup;
-        if (!active) v[0] = v[1] = v[2] = v[3] = (Real)0;
-        seg_sum_n<4>(v, lane, g, NG, red);
-        if (active && g == 0) {
-            const size_t ix = (size_t)(lev - 1) * ncol + col;
-            gpart[ix] = v[0];
-            gpart[n2 + ix] = v[1];
-            gpart[2 * n2 + ix] = v[2];
-            glev[ix] = v[3];
+    __syncthreads();
+    Real a_tb = (Real)0;
+    if (wave == 0) {
+        Real rad[GC], a[GC];
+        const Real top = q.ru(nlay);
+#pragma unroll
+        for (int j = 0; j < GC; ++j) {
+            rad[j] = (Real)0;
+            a[j] = q.live(j, top);
         }
+        // through the sources k, read four layers ahead; the incoming radiances
+        // replace them, the adjoints go to k + 2
+        auto sweep = [&](int first, int step, int k) {
+            Vec tr[4], src[4];
+            Real ct[4];
+            auto fetch = [&](int i, int lev) {
+                tr[i] = at(lev, 1);
+                src[i] = at(lev, k);
+                ct[i] = step < 0 ? q.ru(lev - 1) : lev < nlay ? q.rd(lev) : (Real)0;
+            };
+#pragma unroll
+            for (int i = 0; i < 4; ++i) fetch(i, clampi(first + i * step, 1, nlay));
+            for (int n = 0; n < nlay; n += 4)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (n + i >= nlay) break;
+                    const int lev = first + (n + i) * step;
+                    Vec r, s;
+#pragma unroll
+                    for (int j = 0; j < GC; ++j) {
+                        r.x[j] = rad[j];
+                        s.x[j] = a[j];
+                        rad[j] = fma(src[i].x[j] - rad[j], tr[i].x[j], rad[j]);
+                        a[j] = fma(-a[j], tr[i].x[j], a[j]) + q.live(j, ct[i]);
+                    }
+                    fetch(i, clampi(lev + 4 * step, 1, nlay));
+                    at(lev, k) = r;
+                    at(lev, k + 2) = s;
+                }
+        };
+        sweep(nlay, -1, 2);
+        LwLayer<Real> c;
+        Real fr[GC];
+        u.load(c, 1);
+        u.fracs(c, 1, fr);
+        Vec af;
+        q.surface(fr, rad, a, a_tb, af);
+        *(Vec *)(sums + (size_t)3 * nlay * 64 + lane * GC) = af;
+        sweep(1, 1, 3);
     }
-    {
-        Real v[3];
-        v[0] = active ? pend_up * plkslope(nlay) : (Real)0;
-        v[1] = active ? a_tb : (Real)0;
-        v[2] = active ? a_sec * (Real)dsd : (Real)0;
-        seg_sum_n<3>(v, lane, g, NG, red);
-        if (active && g == 0) {
-            glev[(size_t)nlay * ncol + col] = v[0];
-            gsc[col] = v[1];
-            gsc[ncol + col] = v[2];
+    __syncthreads();
+    for (int lev = 1 + wave; lev <= nlay; lev += WAVES) {
+        Vec rad = at(lev, 3), a = at(lev, 5);
+        if (q.w.bflux) {  // the fluxes: those entering the layer, and those leaving the outermost ones
+            u.store(at(lev, 2).x, lev, 0);
+            u.store(rad.x, lev - 1, 1);
         }
+        const Vec od = at(lev, 0), r = at(lev, 2), s = at(lev, 4);
+        Vec af{};
+        if (lev == 1) af = *(const Vec *)(sums + (size_t)3 * nlay * 64 + lane * GC);
+        LwGroupsD<Real> p;
+        q.load(p, lev);
+        const auto o = q.local(lev, p, od, r, s, af, u.planklev(lev - 1), u.planklev(lev), rad.x, a.x);
+        if (q.w.bflux && lev == nlay) u.store(rad.x, nlay, 1);
+        if (q.w.bflux && lev == 1) {
+            LwLayer<Real> c;
+            Real fr[GC], rad0[GC];
+            u.load(c, 1);
+            u.fracs(c, 1, fr);
+            const Real blay = u.planklay(c), dn = u.planklev(0) - blay;
+#pragma unroll
+            for (int j = 0; j < GC; ++j) {
+                Real atr, tf;
+                u.transmit(od.x[j], atr, tf);
+                rad0[j] = fma(fr[j] * fma(tf, dn, blay) - r.x[j], atr, r.x[j]);
+            }
+            u.store(rad0, 0, 0);
+        }
+        q.store_layer(o, lev);
+        sum(lev, 0) = o.dn;
+        sum(lev, 1) = o.up;
+        sum(lev, 2) = o.sec;
     }
+    __syncthreads();
+    for (int k = wave; k <= nlay; k += WAVES)
+        q.store_level(k == 0 ? sum(1, 0) : k == nlay ? sum(nlay, 1) : sum(k, 1) + sum(k + 1, 0), k);
+    if (wave == 0) {
+        Real a_sec = (Real)0;
+        for (int lev = 1; lev <= nlay; ++lev) a_sec = a_sec + sum(lev, 2);
+        q.store_column(a_tb, a_sec);
+    }
+    __syncthreads();
+}
+
+#pragma clang fp contract(fast)
+
+// the forward's view of the backward's workspace
+__device__ __forceinline__ LwWork lw_vjp_forward(const LwVjpWork &w)
+{
+    LwWork f;
+    f.coef = w.dcoef;
+    f.tlev = w.tlev;
+    f.ipk = w.ipk;
+    f.ilev = w.ilev;
+    f.laytrop = w.laytrop;
+    f.colscal = w.colscal;
+    f.bflux = w.bflux;
+    return f;
 }
 
 // what the LW backward body reads and writes, for the call below
 struct LwUnitArgs {
-    int ncol, nlay, exp_off, tfn_off, plk_off;
+    int ncol, nlay, plk_off;
     gptr<const double> emis, tauaer;  // tauaer NULL: no aerosol
     gptr<const double> colscal;
     gptr<const float> dcoef, dder, tlev, cot, tab;
@@ -323,14 +602,12 @@ struct LwUnitArgs {
     gptr<const LwConst> cst;
     gptr<float> gpart, glev, gsc, bflux;  // bflux NULL: no forward fluxes
 };
-__device__ __forceinline__ LwUnitArgs lw_unit_args(const ColumnInputs &in, const LwVjpWork &w, int exp_off,
-                                                   int tfn_off, int plk_off, const float *tab, const LwConst *cst)
+__device__ __forceinline__ LwUnitArgs lw_unit_args(const ColumnInputs &in, const LwVjpWork &w, int plk_off,
+                                                   const float *tab, const LwConst *cst)
 {
     LwUnitArgs a;
     a.ncol = in.ncol;
     a.nlay = in.nlay;
-    a.exp_off = exp_off;
-    a.tfn_off = tfn_off;
     a.plk_off = plk_off;
     a.emis = (gptr<const double>)in.emis;
     a.tauaer = (gptr<const double>)in.tauaer;
@@ -351,12 +628,14 @@ __device__ __forceinline__ LwUnitArgs lw_unit_args(const ColumnInputs &in, const
     return a;
 }
 
-// The FP32 body with its k-tables in LDS as a function of its own, called by
-// the LW LDS-table backward kernel and by the fused kernel (the same compiled
-// code in both).  s1, s3: the wave's scratch rows.
+// The FP32 body with its tables in LDS, of the LW LDS-table backward kernel and
+// of the fused kernel (a function call of its own: 0.97 ms against 0.95 at
+// 8192 x 40, 5.6 against 5.1 at 32768 x 60).  et: the (exp, tfn)
+// pairs; ktab: the band's k-tables; row: the wave's scratch row; columns c0 on,
+// below cend.
 template <int BAND>
-__device__ __noinline__ void lw_vjp_unit(const LwUnitArgs &a, const LwBand &B, lptr<const float> ktab, WaveUnit u,
-                                         int tile, int lane, gptr<float> s1, gptr<float> s3)
+__device__ __forceinline__ void lw_vjp_unit(const LwUnitArgs &a, const LwBand &B, lptr<const ExpTfn<float>> et,
+                                         lptr<const float> ktab, int c0, int cend, int lane, gptr<float> row)
 {
     ColumnInputs in{};
     in.ncol = a.ncol;
@@ -376,8 +655,26 @@ __device__ __noinline__ void lw_vjp_unit(const LwUnitArgs &a, const LwBand &B, l
     w.glev = (void *)(float *)a.glev;
     w.gsc = (void *)(float *)a.gsc;
     w.bflux = (void *)(float *)a.bflux;
-    lw_vjp_band_body<BAND, float>(in, w, B, (const float *)ktab, (const float *)a.tab, a.exp_off, a.tfn_off,
-                                  a.plk_off, (const LwConst *)a.cst, u, tile, lane, (float *)s1, (float *)s3, nullptr);
+    const LwWork f = lw_vjp_forward(w);
+    const float *tab = (const float *)a.tab, *kt = (const float *)ktab;
+    const LwUnit<BAND, float> u(in, f, B, kt, BAND >= 3 && BAND <= 5 ? tab : kt, tab, (const ExpTfn<float> *)et,
+                                a.plk_off, (const LwConst *)a.cst, c0, cend, lane);
+    lw_vjp_band_body(LwVjpUnit<BAND, float>(u, w), lane, (float *)row);
+}
+// that of band b (0-based)
+__device__ __forceinline__ void lw_vjp_unit_of(const LwUnitArgs &a, const LwBand *bands, int b,
+                                               lptr<const ExpTfn<float>> et, lptr<const float> ktab, int c0, int cend,
+                                               int lane, gptr<float> row)
+{
+#define BODY(bb)                                                                    \
+    case bb - 1:                                                                    \
+        lw_vjp_unit<bb>(a, bands[bb - 1], et, ktab, c0, cend, lane, row);           \
+        break;
+    switch (b) {
+        BODY(1) BODY(2) BODY(3) BODY(4) BODY(5) BODY(6) BODY(7) BODY(8)
+        BODY(9) BODY(10) BODY(11) BODY(12) BODY(13) BODY(14) BODY(15) BODY(16)
+    }
+#undef BODY
 }
 
 }  // namespace rrtmg

@@ -220,7 +220,9 @@ constexpr int der_offset(const unsigned (&mask)[N], int f)
     for (int i = 0; i < f; ++i) o += dmask_count(mask[i]);
     return o;
 }
+// (LW: both in groups of four, [lay][group][col][4], as the forward's)
 constexpr int LW_DSTRIDE = (der_offset(LW_DMASK, LWF_COUNT) + 3) / 4 * 4;
+constexpr int LWD_GROUPS = LW_DSTRIDE / 4;
 constexpr int SW_DSTRIDE = (der_offset(SW_DMASK, SWF_COUNT) + 3) / 4 * 4;
 static_assert(der_offset(LW_DMASK, LWF_COUNT) == 31 && LW_DSTRIDE == 32, "LW derivative record");
 static_assert(der_offset(SW_DMASK, SWF_COUNT) == 17 && SW_DSTRIDE == 20, "SW derivative record");
