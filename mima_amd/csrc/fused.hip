@@ -4,10 +4,10 @@
 // LDS-table backward kernel and of the SW backward band kernel
 // (lw_vjp_body.hpp, sw_vjp_body.hpp); what changes is the schedule: one launch
 // whose workgroups move from LW items to SW items without a kernel boundary,
-// instead of two kernels on two streams.  Measured at 131072 x 60 it is the
-// slower schedule (88.1 against 81.2 ms per forward+backward step): the SW
-// body needs over 168 VGPRs, so the shared kernel runs the LW items at two
-// waves per SIMD where the LW kernel alone runs three.
+// instead of two kernels on two streams.  Measured at 131072 x 60, before the LW
+// body took several g-points a lane, it was the slower schedule (88.1 against
+// 81.2 ms per forward+backward step): the SW body's registers hold the shared
+// kernel at two waves per SIMD.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -1,10 +1,8 @@
 // LW gas optics of one (layer, g-point): per-layer coefficient record, table
-// reader and the 16 band-specialised taumol formulas (rrtmg_lw_taumol.f90).
-// Shared by the forward band kernel and the backward (vector-Jacobian)
-// kernel.  `Real` is the table type; `V` is the arithmetic type of the layer
-// coefficients and results: Real in the forward, a dual number carrying
-// derivatives with respect to layer temperature, water vapour and ozone in
-// the backward.
+// reader and the 16 band-specialised taumol formulas (rrtmg_lw_taumol.f90) of
+// the cloudy band kernels, whose lane is one g-point; the species parameters,
+// transmittances and column sums that all LW kernels share.  `Real` is the
+// table type, `V` the arithmetic type.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -282,9 +280,7 @@ constexpr int lw_chi_ratio_k()
 
 // Optical depth and Planck fraction of one (layer, g) of band BAND,
 // rrtmg_lw_taumol.f90:280-3147.
-// CONST_NSP: the species-parameter counts as compile-time constants (the
-// forward band kernel; the backward's kernels keep the loaded values, as
-// constants they ran 2% slower).
+// CONST_NSP: the species-parameter counts as compile-time constants.
 template <int BAND, typename Real, typename V = Real, bool CONST_NSP = false>
 __device__ __forceinline__ void lw_gas(const LwBand &B, const LTab<Real> &T, const LwConst *__restrict__ cst,
                                        const LwLayer<V> &c, bool lower, V &taug, V &fracs)

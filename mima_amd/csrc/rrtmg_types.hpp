@@ -1,6 +1,7 @@
 // Shared host/device data structures of the gfx950 RRTMG library.
 //
-// Work decomposition (both sides).  Columns are cut into tiles of TILE_COLS
+// Work decomposition of the SW backward and the cloudy kernels (the others:
+// LwLanes, SwLanes).  Columns are cut into tiles of TILE_COLS
 // consecutive columns.  Each one-wave work unit handles one spectral band for
 // up to 64/ng columns of a tile, with lane = (column-in-unit, g-point-in-band),
 // g fastest.  A band's code therefore runs wave-uniformly, table rows of one
